@@ -102,8 +102,8 @@ class Hip:
 # Short names of the forward's kernels (as pgmoe_moe_forward_timed reports their launches).
 _KNAMES = (("router_gemm_kernel", "router"), ("router_logits_kernel", "router"), ("topk_kernel", "topk"),
            ("dispatch_count_kernel", "dispatch_count"), ("identity_dispatch_kernel", "sh_dispatch"),
-           ("dispatch_kernel", "dispatch"), ("gemm_split_reduce_kernel<true>", "gemm_gateup_reduce"),
-           ("gemm_split_reduce_kernel<false>", "gemm_down_reduce"), ("rowscale_kernel", "rowscale"),
+           ("dispatch_kernel", "dispatch"), ("gemm_split_reduce_kernel<1>", "gemm_gateup_reduce"),
+           ("gemm_split_reduce_kernel<0>", "gemm_down_reduce"), ("rowscale_kernel", "rowscale"),
            ("rowscale_block_kernel", "rowscale"),
            ("combine_kernel", "combine"), ("dec_gu_kernel", "dec_gu"), ("dec_dc_kernel", "dec_dc"),
            ("dec_dc_chunk_kernel", "dec_dc"), ("dec_down_kernel", "dec_down"))
@@ -114,7 +114,7 @@ def short_names(raw):
     shared expert's identity dispatch, its products (and its gate's router) get "sh_"."""
     out, shared = [], False
     for r in raw:
-        if "gemm_kernel<" in r:
+        if "gemm_kernel<" in r or "thin_kernel<" in r:
             n = "gemm_gateup" if ", true," in r else "gemm_down"
         else:
             n = next((v for k, v in _KNAMES if k in r), r)

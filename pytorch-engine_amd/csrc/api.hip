@@ -269,19 +269,24 @@ int pgmoe_dense_forward(const pgmoe_dense* D, const uint16_t* x, int32_t M, floa
                                            out, nullptr, 0, st);
         return launch_dec_down_ident(d, WS(float, inter), WS(float, isum), M, out, st);
     }
-    const int BM = gemm_tile_rows();
-    if ((rc = launch_identity_dispatch(M, BM, WS(int32_t, offsets), WS(int32_t, perm), WS(int32_t, inv),
+    const bool tg = thin_takes(g.qtype, M, 1, g.N, g.K, true), td = thin_takes(d.qtype, M, 1, d.N, d.K, false);
+    if ((!tg || !td) &&
+        (rc = launch_identity_dispatch(M, gemm_tile_rows(), WS(int32_t, offsets), WS(int32_t, perm), WS(int32_t, inv),
                                        WS(int32_t, active), WS(int32_t, nact), WS(int32_t, tile_off), WS(float, w),
                                        st)))
         return rc;
-    if ((rc = launch_gateup(g, u, x, M, 1, WS(int32_t, offsets), WS(int32_t, perm), WS(int32_t, active),
-                            WS(int32_t, nact), WS(int32_t, tile_off), 1, WS(float, inter), st, WS(float, raw),
-                            D->act)))
-        return rc;
+    if (tg)  // few rows: no dispatch, row p is token p
+        rc = launch_thin_gateup(g, u, x, M, 1, nullptr, nullptr, nullptr, WS(float, inter), st, WS(float, raw), D->act);
+    else
+        rc = launch_gateup(g, u, x, M, 1, WS(int32_t, offsets), WS(int32_t, perm), WS(int32_t, active),
+                           WS(int32_t, nact), WS(int32_t, tile_off), 1, WS(float, inter), st, WS(float, raw), D->act);
+    if (rc || (rc = launch_rowscale(WS(float, inter), M, d.K, WS(uint16_t, a16), WS(float, rs), st))) return rc;
     // identity order: sorted pair p is token p, so the down rows are the output rows
-    return launch_down(d, WS(float, inter), M, 1, WS(int32_t, offsets), WS(int32_t, perm), WS(int32_t, active),
-                       WS(int32_t, nact), WS(int32_t, tile_off), WS(float, w), 1, WS(uint16_t, a16), WS(float, rs),
-                       out, st, WS(float, raw));
+    if (td)
+        return launch_thin_down(d, WS(uint16_t, a16), WS(float, rs), M, 1, nullptr, nullptr, nullptr, nullptr, out, st,
+                                WS(float, raw));
+    return launch_gemm_down(d, WS(uint16_t, a16), WS(float, rs), M, 1, WS(int32_t, offsets), WS(int32_t, perm),
+                            WS(int32_t, tile_off), WS(float, w), out, st, WS(float, raw));
 #undef WS
 }
 
@@ -456,7 +461,6 @@ static int moe_forward_impl(const pgmoe_layer* L, const LayerMats& lm, const Lay
 #define WS(T, f) reinterpret_cast<T*>(b + o.f)
     const int E = L->n_experts, K = L->top_k, H = L->hidden;
     const int mode = M > decode_tokens_max() ? 1 : 0;
-    const int BM = gemm_tile_rows();
     if (mode == 0) {
         // decode: gate/up with the router and the routing folded in -> [shared gate/up ->
         // shared down] -> down + combine
@@ -504,34 +508,61 @@ static int moe_forward_impl(const pgmoe_layer* L, const LayerMats& lm, const Lay
     }
     if ((rc = launch_router_logits(x, L->router_w, L->router_bias, M, H, E, WS(float, logits), st))) return rc;
     if ((rc = launch_topk(WS(float, logits), M, E, K, L->norm_topk, WS(int32_t, idx), WS(float, w), st))) return rc;
-    if ((rc = launch_dispatch(WS(int32_t, idx), M, K, E, BM, WS(int32_t, offsets), WS(int32_t, perm),
-                              WS(int32_t, inv), WS(int32_t, active), WS(int32_t, nact), WS(int32_t, tile_off), st,
-                              WS(int32_t, dcounts), WS(int32_t, tile_map))))
-        return rc;
-    if ((rc = launch_gateup(lm.gate, lm.up, x, M, K, WS(int32_t, offsets), WS(int32_t, perm), WS(int32_t, active),
-                            WS(int32_t, nact), WS(int32_t, tile_off), mode, WS(float, inter), st, WS(float, raw),
-                            L->act, WS(int32_t, tile_map))))
-        return rc;
-    if ((rc = launch_down(lm.down, WS(float, inter), M, K, WS(int32_t, offsets), WS(int32_t, perm),
-                          WS(int32_t, active), WS(int32_t, nact), WS(int32_t, tile_off), WS(float, w), mode,
-                          WS(uint16_t, a16), WS(float, rs), WS(float, partial), st, WS(float, raw),
-                          WS(int32_t, tile_map))))
-        return rc;
+    const int64_t P = (int64_t)M * K;
+    if (thin_takes(lm.gate.qtype, P, E, lm.gate.N, lm.gate.K, true) &&
+        thin_takes(lm.down.qtype, P, E, lm.down.N, lm.down.K, false)) {  // few pairs an expert
+        if ((rc = launch_dispatch(WS(int32_t, idx), M, K, E, thin_tile_rows(), WS(int32_t, offsets), WS(int32_t, perm),
+                                  WS(int32_t, inv), WS(int32_t, active), WS(int32_t, nact), WS(int32_t, tile_off), st,
+                                  WS(int32_t, dcounts))) ||
+            (rc = launch_thin_gateup(lm.gate, lm.up, x, M, K, WS(int32_t, offsets), WS(int32_t, perm),
+                                     WS(int32_t, tile_off), WS(float, inter), st, WS(float, raw), L->act)) ||
+            (rc = launch_rowscale(WS(float, inter), P, lm.down.K, WS(uint16_t, a16), WS(float, rs), st)) ||
+            (rc = launch_thin_down(lm.down, WS(uint16_t, a16), WS(float, rs), M, K, WS(int32_t, offsets),
+                                   WS(int32_t, perm), WS(int32_t, tile_off), WS(float, w), WS(float, partial), st,
+                                   WS(float, raw))))
+            return rc;
+    } else {
+        if ((rc = launch_dispatch(WS(int32_t, idx), M, K, E, gemm_tile_rows(), WS(int32_t, offsets), WS(int32_t, perm),
+                                  WS(int32_t, inv), WS(int32_t, active), WS(int32_t, nact), WS(int32_t, tile_off), st,
+                                  WS(int32_t, dcounts), WS(int32_t, tile_map))))
+            return rc;
+        if ((rc = launch_gateup(lm.gate, lm.up, x, M, K, WS(int32_t, offsets), WS(int32_t, perm), WS(int32_t, active),
+                                WS(int32_t, nact), WS(int32_t, tile_off), mode, WS(float, inter), st, WS(float, raw),
+                                L->act, WS(int32_t, tile_map))))
+            return rc;
+        if ((rc = launch_down(lm.down, WS(float, inter), M, K, WS(int32_t, offsets), WS(int32_t, perm),
+                              WS(int32_t, active), WS(int32_t, nact), WS(int32_t, tile_off), WS(float, w), mode,
+                              WS(uint16_t, a16), WS(float, rs), WS(float, partial), st, WS(float, raw),
+                              WS(int32_t, tile_map))))
+            return rc;
+    }
     const float* shared = nullptr;
     const float* shared_logit = nullptr;
     if (L->has_shared) {
-        if ((rc = launch_identity_dispatch(M, BM, WS(int32_t, s_offsets), WS(int32_t, s_perm), WS(int32_t, s_inv),
-                                           WS(int32_t, s_active), WS(int32_t, s_nact), WS(int32_t, s_tile_off),
-                                           WS(float, s_w), st)))
+        const bool tg = thin_takes(lm.sg.qtype, M, 1, lm.sg.N, lm.sg.K, true);
+        const bool td = thin_takes(lm.sd.qtype, M, 1, lm.sd.N, lm.sd.K, false);
+        if ((!tg || !td) &&
+            (rc = launch_identity_dispatch(M, gemm_tile_rows(), WS(int32_t, s_offsets), WS(int32_t, s_perm),
+                                           WS(int32_t, s_inv), WS(int32_t, s_active), WS(int32_t, s_nact),
+                                           WS(int32_t, s_tile_off), WS(float, s_w), st)))
             return rc;
-        if ((rc = launch_gateup(lm.sg, lm.su, x, M, 1, WS(int32_t, s_offsets), WS(int32_t, s_perm),
-                                WS(int32_t, s_active), WS(int32_t, s_nact), WS(int32_t, s_tile_off), mode,
-                                WS(float, s_inter), st, WS(float, raw), L->act)))
+        if (tg)
+            rc = launch_thin_gateup(lm.sg, lm.su, x, M, 1, nullptr, nullptr, nullptr, WS(float, s_inter), st,
+                                    WS(float, raw), L->act);
+        else
+            rc = launch_gateup(lm.sg, lm.su, x, M, 1, WS(int32_t, s_offsets), WS(int32_t, s_perm),
+                               WS(int32_t, s_active), WS(int32_t, s_nact), WS(int32_t, s_tile_off), mode,
+                               WS(float, s_inter), st, WS(float, raw), L->act);
+        if (rc || (rc = launch_rowscale(WS(float, s_inter), M, lm.sd.K, WS(uint16_t, s_a16), WS(float, s_rs), st)))
             return rc;
-        if ((rc = launch_down(lm.sd, WS(float, s_inter), M, 1, WS(int32_t, s_offsets), WS(int32_t, s_perm),
-                              WS(int32_t, s_active), WS(int32_t, s_nact), WS(int32_t, s_tile_off), WS(float, s_w),
-                              mode, WS(uint16_t, s_a16), WS(float, s_rs), WS(float, s_partial), st, WS(float, raw))))
-            return rc;
+        if (td)
+            rc = launch_thin_down(lm.sd, WS(uint16_t, s_a16), WS(float, s_rs), M, 1, nullptr, nullptr, nullptr,
+                                  nullptr, WS(float, s_partial), st, WS(float, raw));
+        else
+            rc = launch_gemm_down(lm.sd, WS(uint16_t, s_a16), WS(float, s_rs), M, 1, WS(int32_t, s_offsets),
+                                  WS(int32_t, s_perm), WS(int32_t, s_tile_off), WS(float, s_w), WS(float, s_partial),
+                                  st, WS(float, raw));
+        if (rc) return rc;
         shared = WS(float, s_partial);
         if (L->sh_inp_gate) {
             if ((rc = launch_router_logits(x, L->sh_inp_gate, nullptr, M, H, 1, WS(float, s_logit), st))) return rc;

@@ -209,6 +209,21 @@ int launch_gateup(const Mats& g, const Mats& u, const uint16_t* x, int M, int to
     return launch_gemm_gateup(g, u, x, M, topk, offsets, perm, tile_off, inter, st, raw, act, tile_map);
 }
 
+int launch_rowscale(const float* inter, int64_t P, int I, uint16_t* a16, float* rs, hipStream_t st) {
+    const dim3 rgrid(div_up(P, 4));  // I: a multiple of 256 (checked with the weights)
+    if (I <= 1024)
+        PG_LAUNCH(rowscale_kernel<4>, rgrid, dim3(256), 0, st, inter, (int)P, I, a16, rs);
+    else if (I <= 4096)
+        PG_LAUNCH(rowscale_kernel<16>, rgrid, dim3(256), 0, st, inter, (int)P, I, a16, rs);
+    else if (I <= 16384)
+        PG_LAUNCH(rowscale_block_kernel<16>, dim3((unsigned)P), dim3(256), 0, st, inter, I, a16, rs);
+    else if (I <= 24576)
+        PG_LAUNCH(rowscale_block_kernel<24>, dim3((unsigned)P), dim3(256), 0, st, inter, I, a16, rs);
+    else
+        PG_LAUNCH(rowscale_kernel<0>, rgrid, dim3(256), 0, st, inter, (int)P, I, a16, rs);
+    return check_launch("rowscale");
+}
+
 int launch_down(const Mats& d, const float* inter, int M, int topk, const int32_t* offsets, const int32_t* perm,
                 const int32_t* active, const int32_t* n_active, const int32_t* tile_off, const float* topk_w,
                 int mode, uint16_t* a16, float* rs, float* partial, hipStream_t st, float* raw,
@@ -220,19 +235,7 @@ int launch_down(const Mats& d, const float* inter, int M, int topk, const int32_
         return launch_dec_down(d, inter, nullptr, M, offsets, perm, active, n_active, (int)(P < E ? P : E), topk_w,
                                partial, st);
     if (!a16 || !rs) return fail(PGMOE_E_INVALID, "GEMM mode needs a16 and rs scratch");
-    const int I = d.K;  // a multiple of 256 (checked with the weights)
-    const dim3 rgrid(div_up(P, 4));
-    if (I <= 1024)
-        PG_LAUNCH(rowscale_kernel<4>, rgrid, dim3(256), 0, st, inter, (int)P, I, a16, rs);
-    else if (I <= 4096)
-        PG_LAUNCH(rowscale_kernel<16>, rgrid, dim3(256), 0, st, inter, (int)P, I, a16, rs);
-    else if (I <= 16384)
-        PG_LAUNCH(rowscale_block_kernel<16>, dim3((unsigned)P), dim3(256), 0, st, inter, I, a16, rs);
-    else if (I <= 24576)
-        PG_LAUNCH(rowscale_block_kernel<24>, dim3((unsigned)P), dim3(256), 0, st, inter, I, a16, rs);
-    else
-        PG_LAUNCH(rowscale_kernel<0>, rgrid, dim3(256), 0, st, inter, (int)P, I, a16, rs);
-    int rc = check_launch("rowscale");
+    int rc = launch_rowscale(inter, P, d.K, a16, rs, st);
     if (rc) return rc;
     return launch_gemm_down(d, a16, rs, M, topk, offsets, perm, tile_off, topk_w, partial, st, raw, tile_map);
 }

@@ -1,4 +1,4 @@
-// Prefill (M > 8) grouped expert products on the MFMA cores.
+// Prefill (M > 8) grouped expert products on the MFMA cores (few pairs an expert: thin.hip).
 //
 // A tile is 256 sorted pairs of one expert x 256 output columns.  The gate/up block is 8
 // waves (two per SIMD; each owns 128 rows x 64 columns, so each B column is decoded by the
@@ -706,12 +706,15 @@ __global__ __launch_bounds__(64 * (WM * 8 / CT)) void gemm_kernel(
 // the same order run at streaming rate.  Measured (Qwen2 shared expert's down product,
 // M = 512): one column a thread 17.3 us, four 13.2 us.
 constexpr int kMaxSplitLoads = 8;
-template <bool GATEUP>
+// KIND 0: down, 1: gate/up, 2: linear (rs = the bias or null, act = fp16 output).
+template <int KIND>
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const float* __restrict__ raw, int S, int64_t P,
                                                                 int N, const float* __restrict__ rs,
                                                                 const float* __restrict__ topk_w,
                                                                 const int32_t* __restrict__ perm,
-                                                                float* __restrict__ out, int act) {
+                                                                void* __restrict__ outv, int act) {
+    constexpr bool GATEUP = KIND == 1;
+    float* out = (float*)outv;
     const int N4 = N >> 2;
     const int64_t n4 = P * N4;
     const int NC = GATEUP ? 2 * N : N;
@@ -752,9 +755,17 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const float* __r
         if constexpr (GATEUP) {
             o = make_float4(act_fast(act, a.x) * b.x, act_fast(act, a.y) * b.y, act_fast(act, a.z) * b.z,
                             act_fast(act, a.w) * b.w);
-        } else {
-            const float f = rs[p] * topk_w[perm[p]];
+        } else if constexpr (KIND == 0) {
+            const float f = topk_w ? rs[p] * topk_w[perm[p]] : rs[p];
             o = make_float4(f * a.x, f * a.y, f * a.z, f * a.w);
+        } else {
+            const float4 b4 = rs ? make_float4(rs[c], rs[c + 1], rs[c + 2], rs[c + 3]) : make_float4(0.f, 0.f, 0.f, 0.f);
+            o = make_float4(a.x + b4.x, a.y + b4.y, a.z + b4.z, a.w + b4.w);
+            if (act) {
+                typedef half_t h4 __attribute__((ext_vector_type(4), aligned(4)));
+                *(h4*)((half_t*)outv + p * N + c) = h4{(half_t)o.x, (half_t)o.y, (half_t)o.z, (half_t)o.w};
+                continue;
+            }
         }
         *(float4*)(out + p * N + c) = o;
     }
@@ -828,17 +839,17 @@ size_t gemm_split_bytes_upto(int64_t P, int E, int N, int K, bool gateup) {
     return best;
 }
 
-static int launch_split_reduce(bool gateup, const float* raw, int S, int64_t P, int N, const float* rs,
-                               const float* topk_w, const int32_t* perm, float* out, hipStream_t st, int act) {
+int launch_split_reduce(int kind, const float* raw, int S, int64_t P, int N, const float* rs, const float* topk_w,
+                        const int32_t* perm, void* out, hipStream_t st, int act) {
     const int64_t n = P * (N / 4);  // four columns a thread
     const int blocks = (int)(div_up(n, 256) < 16384 ? div_up(n, 256) : 16384);
     if (N % 4) return fail(PGMOE_E_UNSUPPORTED, "split reduce: N %d is not a multiple of 4", N);
-    if (gateup)
-        PG_LAUNCH(gemm_split_reduce_kernel<true>, dim3(blocks), dim3(256), 0, st, raw, S, P, N, rs, topk_w, perm, out,
-                  act);
-    else
-        PG_LAUNCH(gemm_split_reduce_kernel<false>, dim3(blocks), dim3(256), 0, st, raw, S, P, N, rs, topk_w, perm, out,
-                  act);
+#define PG_SR(KIND) \
+    PG_LAUNCH(gemm_split_reduce_kernel<KIND>, dim3(blocks), dim3(256), 0, st, raw, S, P, N, rs, topk_w, perm, out, act)
+    if (kind == 1) PG_SR(1);
+    else if (kind == 0) PG_SR(0);
+    else PG_SR(2);
+#undef PG_SR
     return check_launch("gemm split reduce");
 }
 
@@ -900,7 +911,7 @@ int launch_gemm_gateup(const Mats& g, const Mats& u, const uint16_t* x, int M, i
 #undef PG_GU
     int rc = check_launch("gemm_gateup");
     if (rc || sp.ksplit == 1) return rc;
-    return launch_split_reduce(true, raw, sp.ksplit, P, g.N, nullptr, nullptr, nullptr, inter, st, act);
+    return launch_split_reduce(1, raw, sp.ksplit, P, g.N, nullptr, nullptr, nullptr, inter, st, act);
 }
 
 int launch_gemm_down(const Mats& d, const uint16_t* a16, const float* rs, int M, int topk, const int32_t* offsets,
@@ -930,7 +941,7 @@ int launch_gemm_down(const Mats& d, const uint16_t* a16, const float* rs, int M,
 #undef PG_DN
     int rc = check_launch("gemm_down");
     if (rc || sp.ksplit == 1) return rc;
-    return launch_split_reduce(false, raw, sp.ksplit, P, d.N, rs, topk_w, perm, partial, st, PGMOE_ACT_SILU);
+    return launch_split_reduce(0, raw, sp.ksplit, P, d.N, rs, topk_w, perm, partial, st, PGMOE_ACT_SILU);
 }
 
 }  // namespace pgmoe

@@ -66,6 +66,8 @@ int launch_down(const Mats& d, const float* inter, int M, int topk, const int32_
                 int mode, uint16_t* a16, float* rs, float* partial, hipStream_t st, float* raw = nullptr,
                 const int32_t* tile_map = nullptr);
 // clear (optional): n_clear words the kernel sets to zero (the decode router's tagged logits).
+// The row-scaled fp16 down input (a16, rs) of P fp32 rows of I values.
+int launch_rowscale(const float* inter, int64_t P, int I, uint16_t* a16, float* rs, hipStream_t st);
 int launch_combine(const float* partial, const int32_t* inv, int M, int K, int H, const float* shared,
                    const float* shared_logit, float* out, hipStream_t st, uint64_t* clear = nullptr,
                    int n_clear = 0);
@@ -161,6 +163,23 @@ size_t gemm_split_bytes(int64_t P, int E, int N, int K, bool gateup);
 // to P pairs must hold).
 size_t gemm_split_bytes_upto(int64_t P, int E, int N, int K, bool gateup);
 int gemm_tile_pairs();
+// The S raw partial sums [split][P][N] (gate/up: 2N) added in split order, then the epilogue
+// of kind 0 (down), 1 (gate/up, act) or 2 (linear: rs = bias or null, act = fp16 output).
+int launch_split_reduce(int kind, const float* raw, int S, int64_t P, int N, const float* rs, const float* topk_w,
+                        const int32_t* perm, void* out, hipStream_t st, int act);
+// Products of few rows an expert (thin.hip), on tiles of thin_tile_rows() pairs; the same
+// arguments as the grouped GEMMs (tile_off counts thin tiles).  offsets, perm, tile_off and
+// topk_w null: one matrix, pair p is row p with weight 1.  raw: split-K scratch of the
+// grouped GEMM's size, or null.
+bool thin_takes(int qtype, int64_t P, int E, int N, int K, bool gateup);
+int thin_tile_rows();
+int launch_thin_gateup(const Mats& g, const Mats& u, const uint16_t* x, int M, int topk, const int32_t* offsets,
+                       const int32_t* perm, const int32_t* tile_off, float* inter, hipStream_t st, float* raw, int act);
+int launch_thin_down(const Mats& d, const uint16_t* a16, const float* rs, int M, int topk, const int32_t* offsets,
+                     const int32_t* perm, const int32_t* tile_off, const float* topk_w, float* partial,
+                     hipStream_t st, float* raw);
+int launch_thin_linear(const Mats& w, const uint16_t* x, int M, const float* bias, void* out, int out_f16, float* raw,
+                       hipStream_t st);
 int64_t layout_bytes(int qtype, int64_t rows, int64_t cols);
 // Scale plane (relayout.hip): bytes of one matrix's plane (0 for Q8_0, -1 if unsupported)
 // and its load-time construction from the device layout.

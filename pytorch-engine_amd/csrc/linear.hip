@@ -5,8 +5,10 @@
 // GGUFQuantLinear.embed_lookup (:1839-1863).
 //   M <= 8 : the decode GEMV in its single-matrix mode (dec_gu_kernel<..., kLinear>), bias
 //            and output rounding in its epilogue;
-//   M  > 8 : identity dispatch, then the grouped MFMA GEMM (the down product's form, A = x
-//            read directly, unit row scales), then a bias / fp16 pass when asked for.
+//   M  > 8 : thin tiles (thin.hip; bias and rounding in their epilogue or split reduce) up to
+//            a few hundred rows, else identity dispatch, the grouped MFMA GEMM (the down
+//            product's form, A = x read directly, unit row scales) and a bias / fp16 pass when
+//            asked for.
 #include "decode_kernels.h"
 
 namespace pgmoe {
@@ -156,6 +158,7 @@ int launch_linear(const Mats& w, const float* bias, const uint16_t* x, int M, vo
     float* prod = staged ? (float*)take((size_t)M * w.N * 4) : (float*)out;
     const size_t rb = gemm_split_bytes(M, 1, w.N, w.K, false);
     float* raw = rb ? (float*)take(rb) : nullptr;
+    if (thin_takes(w.qtype, M, 1, w.N, w.K, false)) return launch_thin_linear(w, x, M, bias, out, out_f16, raw, st);
     int rc = launch_identity_dispatch(M, gemm_tile_rows(), offsets, perm, inv, active, nact, tile_off, ones, st);
     if (rc) return rc;
     // the down GEMM's epilogue scales row p by rs[p] * topk_w[perm[p]]: both 1 here

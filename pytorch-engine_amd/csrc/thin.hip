@@ -1,0 +1,792 @@
+// Grouped products of few rows an expert (9 .. a few hundred tokens): the weights are
+// streamed once, straight from HBM into registers, and every token of a tile shares them.
+//
+// A tile is up to 32 sorted pairs of one expert (64 rows of a linear).  A block of 8 waves
+// takes one tile and 8 row tiles of 16 weight rows (gate/up: 8 of gate and the same 8 of up,
+// both in the same wave), and walks the whole K range or a split of it.  Lane (r, p) of a
+// wave owns row r's quarter p (64 weights) of each 256-weight super-block, as in the decode
+// GEMVs: 16-byte loads of whole 256-byte row runs, the quarter's own scales decoded once,
+// no weight bytes through LDS.  A k step of v_mfma_f32_16x16x32_f16 takes 8 weights of each
+// quarter (the order of k inside a product is free as long as both operands agree), so a
+// super-block is 8 steps of 16 tokens x 16 rows.  The tokens' fp16 rows are the other
+// operand: staged through two LDS buffers, one stage ahead of its use and a super-block's
+// share at a time, with as many super-blocks a stage as the tile's rows leave room for.
+//
+// Against the 256 x 256 tiles of gemm.hip, which one expert's few rows leave nearly empty:
+// no decoded scale plane is read (44 % more bytes than Q4_K's own), two blocks share a CU, so
+// loads stay in flight across the barriers, and 16 tokens cost 16 rows of MFMA.
+//
+// What bounds it: the weight stream.  Mixtral-shaped gate/up, 24 tokens (529 MB of Q4_K): 209
+// us on the 256-row tiles, 111-116 here (4.6-4.8 TB/s); 97 us with the loads alone (5.4 TB/s, the
+// products and decode taken out of a copy), so the VALU work is nearly hidden.  Qwen3 shape, 32
+// tokens: gate/up 84 -> 42 us, down 58 -> 33; H = 4096, I = 12288 FFN of 20 rows 74 -> 44 us;
+// 4096 x 6144 Q4_K linear of 33 rows 25 -> 18.6 us.  Tried and slower: two K halves in one
+// block (shorter units, no better end: 43 -> 47 us), 64-pair tiles with one row tile a wave for
+// gate/up (102 -> 106 us a layer; the tokens are staged twice as often), weights requested two
+// super-blocks ahead (3-5 %).
+// Reference: GGUFQuantMoEExperts.forward_expert (quant_kernels.py:1990-2011) ->
+// exec_w4a16_matmul / exec_w8a16_matmul (:1165-1420) and model.py:916-919.
+#include <algorithm>
+
+#include "common.h"
+#include "decode_kernels.h"
+#include "launch.h"
+
+namespace pgmoe {
+
+#ifndef PG_THIN_R
+#define PG_THIN_R 1
+#endif
+constexpr int kThinRows = 64;  // most pairs a tile
+constexpr int kThinWaves = 8;
+constexpr int kThinThreads = 64 * kThinWaves;
+constexpr int kThinSums = 64 * 80;  // bytes of a stage's sub-block sums
+constexpr int kThinStage = kThinRows * (512 + 16);  // bytes of an LDS stage (any rows x super-blocks split)
+
+typedef _Float16 th8 __attribute__((ext_vector_type(8)));
+typedef _Float16 th2 __attribute__((ext_vector_type(2)));
+typedef __bf16 tb8 __attribute__((ext_vector_type(8)));
+typedef float tf4 __attribute__((ext_vector_type(4)));
+
+// ---------------------------------------------------------------- weight decode
+// Each lane turns its quarter's codes into fp16 MFMA operands with packed fp16 arithmetic
+// (4 cycles for two weights; v_fma_mixlo / mixhi_f16 take 8 each, v_fma_mix_f32 and
+// v_cvt_pk_f16_f32 4 each) that is exact, or rounds as the fp32 form would:
+//   Q4_K, Q5_K: sc q (an integer below 2048, exact); the products of a super-block are summed
+//               unscaled and then take d in fp32 (POST); the minima are a second product, of
+//               the 6-bit m and the tokens' fp32 sums over each sub-block as three bf16 pieces
+//               (their 24 bits, so exact as well), which takes dmin in fp32 (MINS);
+//   Q6_K      : sc (q - 32), rounded once above 2048; d in fp32 (POST);
+//   Q8_0      : d q, rounded once (the bits of the fp32 product rounded to fp16);
+//   Q4_1      : d q + m in fp32, rounded once (d and m are fp16: no integer form);
+//   F16       : as stored.
+__device__ __forceinline__ th2 as_h2(uint32_t v) { return __builtin_bit_cast(th2, v); }
+__device__ __forceinline__ th2 h2(float v) { return th2{(_Float16)v, (_Float16)v}; }
+__device__ __forceinline__ th2 pk_fma(th2 a, th2 b, th2 c) { return __builtin_elementwise_fma(a, b, c); }
+__device__ __forceinline__ th8 cat8(const th2 (&v)[4]) {
+    return th8{v[0].x, v[0].y, v[1].x, v[1].y, v[2].x, v[2].y, v[3].x, v[3].y};
+}
+
+// Constants of the decode held in registers: v_and_or_b32 takes no literal, and one scalar.
+struct ThinConst {
+    uint32_t magic, mask, mask2;  // 0x6400 twice (fp16 1024); code masks of byte pairs
+    uint32_t sh, sd, md, ml;      // header shifts and masks of a K-quant lane's quarter (thin_kscales)
+};
+template <int QT>
+__device__ __forceinline__ ThinConst thin_const(int p) {
+    ThinConst k{};
+    k.magic = 0x64006400u;
+    k.mask = QT == PGMOE_Q5_K ? 0x001f001fu : QT == PGMOE_Q6_K ? 0x003f003fu : 0x000f000fu;
+    k.mask2 = 0x00f000f0u;
+    asm("" : "+v"(k.magic));
+    asm("" : "+s"(k.mask));
+    asm("" : "+s"(k.mask2));
+    if constexpr (QT == PGMOE_Q4_K || QT == PGMOE_Q5_K) {
+        k.sh = 16 * (p & 1);
+        k.sd = k.sh + (p < 2 ? 0 : 2);
+        k.md = p < 2 ? 0x3f3fu : 0x3030u;
+        k.ml = p < 2 ? 0u : 0x0f0fu;
+    }
+    if constexpr (QT == PGMOE_Q6_K) k.sh = 8 * (p & 1);
+    return k;
+}
+
+// Codes 0 and 2, then 1 and 3, of a word's bytes under `mask` as fp16 pairs 1024 + (byte &
+// mask): one v_and_or_b32 a pair.  The staged activations have the same order inside every
+// four elements (thin_permute).
+__device__ __forceinline__ void thin_codes(const ThinConst& k, uint32_t w, uint32_t mask, th2& m0, th2& m1) {
+    m0 = as_h2((w & mask) | k.magic);
+    m1 = as_h2(((w >> 8) & mask) | k.magic);
+}
+__device__ __forceinline__ uint32_t thin_bfi(uint32_t mask, uint32_t a, uint32_t b) { return (mask & a) | (~mask & b); }
+
+// A lane's quarter: pair(i), i = 0..3, gives the 8-weight fragments of two k steps;
+// elem(i, half) is a fragment's first element, from base(p).
+template <int QT> struct ThinW;
+
+// (scale, min) of sub-blocks 2p (low byte) and 2p + 1 from a K-quant header: for p < 2 six bits
+// of D's and Mb's bytes, else the nibbles of MD's bytes with the top two bits of D's and Mb's.
+__device__ __forceinline__ void thin_kscales(const ThinConst& k, const u32x4& h, uint32_t& sc, uint32_t& mn) {
+    sc = ((h.y >> k.sd) & k.md) | ((h.w >> k.sh) & k.ml);
+    mn = ((h.z >> k.sd) & k.md) | ((h.w >> (k.sh + 4)) & k.ml);
+}
+struct ThinK {  // the header of Q4_K and Q5_K
+    static constexpr bool POST = true, MINS = true;
+    uint32_t ddm, mn;  // d and dmin (fp16); the minima of sub-blocks 2p, 2p + 1 (bytes)
+    th2 s0, s1;        // their scales, twice
+    __device__ __forceinline__ ThinK(const ThinConst& kc, const u32x4& h) {
+        uint32_t sc;
+        thin_kscales(kc, h, sc, mn);
+        ddm = h.x;
+        s0 = as_h2(__builtin_amdgcn_perm(kc.magic, sc, 0x05000500u)) - h2(1024.0f);
+        s1 = as_h2(__builtin_amdgcn_perm(kc.magic, sc, 0x05010501u)) - h2(1024.0f);
+    }
+    __device__ __forceinline__ float scale() const { return lo_half(ddm); }
+    __device__ __forceinline__ float min_scale() const { return hi_half(ddm); }
+    __device__ __forceinline__ tb8 mins() const {  // each minimum (6 bits, exact) against three pieces of its sum
+        const uint32_t f0 = __builtin_bit_cast(uint32_t, (float)(mn & 0xff));
+        const uint32_t f1 = __builtin_bit_cast(uint32_t, (float)((mn >> 8) & 0xff));
+        const uint32_t a = __builtin_amdgcn_perm(f0, f0, 0x03020302u), b = __builtin_amdgcn_perm(f1, f1, 0x03020302u);
+        return __builtin_bit_cast(tb8, u32x4{a, a, b, b});
+    }
+    __device__ static __forceinline__ constexpr int elem(int i, int half) { return 8 * i + 32 * half; }
+    __device__ static __forceinline__ int base(int p) { return 64 * p; }
+};
+template <> struct ThinW<PGMOE_Q4_K> : ThinK {
+    uint32_t w[8];
+    th2 c0, c1;
+    __device__ __forceinline__ ThinW(const ThinConst& kc, const Qtr<PGMOE_Q4_K>& q) : ThinK(kc, q.h) {
+        w[0] = q.a.x, w[1] = q.a.y, w[2] = q.a.z, w[3] = q.a.w;
+        w[4] = q.b.x, w[5] = q.b.y, w[6] = q.b.z, w[7] = q.b.w;
+        s1 = s1 * h2(0.0625f);  // the high nibbles are read in place, as 1024 + 16 q
+        c0 = s0 * h2(-1024.0f);
+        c1 = s1 * h2(-1024.0f);
+    }
+    __device__ __forceinline__ void pair(const ThinConst& kc, int i, th8& lo, th8& hi) const {
+        th2 m[4], n[4];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            thin_codes(kc, w[2 * i + k], kc.mask, m[2 * k], m[2 * k + 1]);
+            thin_codes(kc, w[2 * i + k], kc.mask2, n[2 * k], n[2 * k + 1]);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            m[k] = pk_fma(m[k], s0, c0);
+            n[k] = pk_fma(n[k], s1, c1);
+        }
+        lo = cat8(m);
+        hi = cat8(n);
+    }
+};
+template <> struct ThinW<PGMOE_Q5_K> : ThinK {
+    uint32_t w[8], hx, hy;
+    th2 c0, c1;
+    __device__ __forceinline__ ThinW(const ThinConst& kc, const Qtr<PGMOE_Q5_K>& q) : ThinK(kc, q.h) {
+        w[0] = q.a.x, w[1] = q.a.y, w[2] = q.a.z, w[3] = q.a.w;
+        w[4] = q.b.x, w[5] = q.b.y, w[6] = q.b.z, w[7] = q.b.w;
+        hx = q.hb.x;
+        hy = q.hb.y;
+        c0 = s0 * h2(-1024.0f);
+        c1 = s1 * h2(-1024.0f);
+    }
+    __device__ __forceinline__ void pair(const ThinConst& kc, int i, th8& lo, th8& hi) const {
+        th2 m[4], n[4];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {  // word j: the fifth bits of its four elements are bits j + 8b of hx / hy
+            const int j = 2 * i + k;
+            const uint32_t bx = j < 4 ? hx << (4 - j) : hx >> (j - 4), by = j < 4 ? hy << (4 - j) : hy >> (j - 4);
+            thin_codes(kc, thin_bfi(0x10101010u, bx, w[j]), kc.mask, m[2 * k], m[2 * k + 1]);
+            thin_codes(kc, thin_bfi(0x10101010u, by, w[j] >> 4), kc.mask, n[2 * k], n[2 * k + 1]);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            m[k] = pk_fma(m[k], s0, c0);
+            n[k] = pk_fma(n[k], s1, c1);
+        }
+        lo = cat8(m);
+        hi = cat8(n);
+    }
+};
+template <> struct ThinW<PGMOE_Q6_K> {
+    static constexpr bool POST = true, MINS = false;
+    float d;
+    __device__ __forceinline__ float scale() const { return d; }
+    th2 s01, s23;  // scales of sub-blocks s = 0, 1 and 2, 3
+    uint32_t la[4], lb[4], qh[4];
+    __device__ __forceinline__ ThinW(const ThinConst& kc, const Qtr<PGMOE_Q6_K>& q) {
+        d = h2f((uint16_t)q.d);
+        s01 = as_h2((((q.sc.x >> kc.sh) & 0x00ff00ffu) ^ 0x00800080u) | kc.magic) - h2(1152.0f);
+        s23 = as_h2((((q.sc.y >> kc.sh) & 0x00ff00ffu) ^ 0x00800080u) | kc.magic) - h2(1152.0f);
+        la[0] = q.la.x, la[1] = q.la.y, la[2] = q.la.z, la[3] = q.la.w;
+        lb[0] = q.lb.x, lb[1] = q.lb.y, lb[2] = q.lb.z, lb[3] = q.lb.w;
+        qh[0] = q.qh.x, qh[1] = q.qh.y, qh[2] = q.qh.z, qh[3] = q.qh.w;
+    }
+    // step pair i: chunk la (i even) or lb, its first or second 8 bytes; sub-blocks s = i & 1
+    // (low nibbles) and s + 2 (high), high bits 2s of each qh byte
+    __device__ __forceinline__ void pair(const ThinConst& kc, int i, th8& lo, th8& hi) const {
+        th2 m[4], n[4];
+        const int s = i & 1;
+        const th2 a = s ? th2{s01.y, s01.y} : th2{s01.x, s01.x}, b = s ? th2{s23.y, s23.y} : th2{s23.x, s23.x};
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int j = 2 * (i >> 1) + k;
+            const uint32_t l = s ? lb[j] : la[j], h = qh[j];
+            thin_codes(kc, thin_bfi(0x30303030u, s ? h << 2 : h << 4, l), kc.mask, m[2 * k], m[2 * k + 1]);
+            thin_codes(kc, thin_bfi(0x30303030u, s ? h >> 2 : h, l >> 4), kc.mask, n[2 * k], n[2 * k + 1]);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            m[k] = (m[k] - h2(1056.0f)) * a;
+            n[k] = (n[k] - h2(1056.0f)) * b;
+        }
+        lo = cat8(m);
+        hi = cat8(n);
+    }
+    __device__ static __forceinline__ constexpr int elem(int i, int half) {
+        return 32 * (i & 1) + 8 * (i >> 1) + 64 * half;
+    }
+    __device__ static __forceinline__ int base(int p) { return 128 * (p >> 1) + 16 * (p & 1); }
+};
+template <> struct ThinW<PGMOE_Q8_0> {
+    static constexpr bool POST = false, MINS = false;
+    th2 dd;  // d of blocks 2p, 2p + 1
+    u32x4 c[4];
+    __device__ __forceinline__ ThinW(const ThinConst&, const Qtr<PGMOE_Q8_0>& q) {
+        dd = as_h2(q.d);
+        c[0] = q.c0, c[1] = q.c1, c[2] = q.c2, c[3] = q.c3;
+    }
+    __device__ __forceinline__ void pair(const ThinConst& kc, int i, th8& lo, th8& hi) const {
+        const th2 a = i < 2 ? th2{dd.x, dd.x} : th2{dd.y, dd.y};
+        const uint32_t v[4] = {c[i].x ^ 0x80808080u, c[i].y ^ 0x80808080u, c[i].z ^ 0x80808080u, c[i].w ^ 0x80808080u};
+        th2 m[4], n[4];  // 1152 + q, bytes (0, 2) and (1, 3) of each word
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            m[2 * k] = as_h2(__builtin_amdgcn_perm(kc.magic, v[k], 0x05020500u));
+            m[2 * k + 1] = as_h2(__builtin_amdgcn_perm(kc.magic, v[k], 0x05030501u));
+            n[2 * k] = as_h2(__builtin_amdgcn_perm(kc.magic, v[2 + k], 0x05020500u));
+            n[2 * k + 1] = as_h2(__builtin_amdgcn_perm(kc.magic, v[2 + k], 0x05030501u));
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            m[k] = (m[k] - h2(1152.0f)) * a;
+            n[k] = (n[k] - h2(1152.0f)) * a;
+        }
+        lo = cat8(m);
+        hi = cat8(n);
+    }
+    __device__ static __forceinline__ constexpr int elem(int i, int half) { return 16 * i + 8 * half; }
+    __device__ static __forceinline__ int base(int p) { return 64 * p; }
+};
+template <> struct ThinW<PGMOE_Q4_1> {
+    static constexpr bool POST = false, MINS = false;
+    float a0, c0, a1, c1;
+    uint32_t w[8];
+    __device__ __forceinline__ ThinW(const ThinConst&, const Qtr<PGMOE_Q4_1>& q) {
+        a0 = lo_half(q.dw);
+        c0 = lo_half(q.mw) - 1024.0f * a0;
+        const float a = hi_half(q.dw);
+        c1 = hi_half(q.mw) - 64.0f * a;
+        a1 = a * 0.0625f;
+        w[0] = q.a.x, w[1] = q.a.y, w[2] = q.a.z, w[3] = q.a.w;
+        w[4] = q.b.x, w[5] = q.b.y, w[6] = q.b.z, w[7] = q.b.w;
+    }
+    __device__ __forceinline__ static th2 deq(th2 v, float a, float c) {
+        return th2{(_Float16)__builtin_fmaf((float)v.x, a, c), (_Float16)__builtin_fmaf((float)v.y, a, c)};
+    }
+    __device__ __forceinline__ void pair(const ThinConst& kc, int i, th8& lo, th8& hi) const {
+        th2 m[4], n[4];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            thin_codes(kc, w[2 * i + k], kc.mask, m[2 * k], m[2 * k + 1]);
+            thin_codes(kc, w[2 * i + k], kc.mask2, n[2 * k], n[2 * k + 1]);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            m[k] = deq(m[k], a0, c0);
+            n[k] = deq(n[k], a1, c1);
+        }
+        lo = cat8(m);
+        hi = cat8(n);
+    }
+    __device__ static __forceinline__ constexpr int elem(int i, int half) { return 8 * i + 32 * half; }
+    __device__ static __forceinline__ int base(int p) { return 64 * p; }
+};
+template <> struct ThinW<PGMOE_F16> {
+    static constexpr bool POST = false, MINS = false;
+    u32x4 c[8];
+    __device__ __forceinline__ ThinW(const ThinConst&, const Qtr<PGMOE_F16>& q) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) c[i] = q.c[i];
+    }
+    __device__ __forceinline__ void pair(const ThinConst&, int i, th8& lo, th8& hi) const {
+        lo = __builtin_bit_cast(th8, c[2 * i]);
+        hi = __builtin_bit_cast(th8, c[2 * i + 1]);
+    }
+    __device__ static __forceinline__ constexpr int elem(int i, int half) { return 16 * i + 8 * half; }
+    __device__ static __forceinline__ int base(int p) { return 64 * p; }
+};
+
+// 8 activations in thin_codes' order: elements 0, 2, 1, 3 of each four.
+template <int QT>
+__device__ __forceinline__ u32x4 thin_permute(u32x4 v) {
+    if constexpr (QT == PGMOE_F16) return v;
+    u32x4 r;
+    r.x = __builtin_amdgcn_perm(v.y, v.x, 0x05040100u);
+    r.y = __builtin_amdgcn_perm(v.y, v.x, 0x07060302u);
+    r.z = __builtin_amdgcn_perm(v.w, v.z, 0x05040100u);
+    r.w = __builtin_amdgcn_perm(v.w, v.z, 0x07060302u);
+    return r;
+}
+
+__device__ __forceinline__ float thin_act(int act, float g) {  // gemm.hip's hardware exp2 / reciprocal forms
+    const float z = 0.7978845608028654f * (g + 0.044715f * g * g * g);
+    return act ? g - g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(2.8853900817779268f * z))
+               : g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g));
+}
+
+// Quarter loads of super-block tile t (wave-uniform, at the row tile's first row): the lane
+// part of every address is one of two 32-bit offsets, off0 (the row's 16 bytes) and offp (the
+// quarter's first chunk of them); d: the row tile's d plane position (Q6_K).
+template <int QT>
+__device__ __forceinline__ void thin_offsets(int lane, int p, uint32_t& off0, uint32_t& offp) {
+    off0 = (lane & 15) * 16;
+    offp = off0;
+    if constexpr (QT == PGMOE_Q4_K || QT == PGMOE_Q5_K) offp += (1 + 2 * p) * 1024;
+    else if constexpr (QT == PGMOE_Q4_1) offp += (2 + 2 * p) * 1024;
+    else if constexpr (QT == PGMOE_Q6_K) offp += (4 * (p >> 1) + (p & 1)) * 1024;
+    else if constexpr (QT == PGMOE_Q8_0) offp += 4 * p * 1024;
+    else offp += 8 * p * 1024;
+}
+template <int QT>
+__device__ __forceinline__ void thin_load(Qtr<QT>& q, const uint8_t* t, const uint8_t* d, uint32_t off0, uint32_t offp,
+                                          int lane, int p) {
+    if constexpr (QT == PGMOE_Q4_1) {
+        q.dw = *(const uint32_t*)(t + (off0 + 4 * p));
+        q.mw = *(const uint32_t*)(t + (off0 + 4 * p) + 1024);
+        q.a = ldq(t + offp);
+        q.b = ldq(t + offp + 1024);
+    } else if constexpr (QT == PGMOE_Q4_K || QT == PGMOE_Q5_K) {
+        q.h = ldq(t + off0);
+        q.a = ldq(t + offp);
+        q.b = ldq(t + offp + 1024);
+        if constexpr (QT == PGMOE_Q5_K) q.hb = *(const u32x2*)(t + (off0 + (9 + (p >> 1)) * 1024 + 8 * (p & 1)));
+    } else if constexpr (QT == PGMOE_Q6_K) {
+        q.la = ldq(t + offp);
+        q.lb = ldq(t + offp + 2048);
+        q.qh = ldq(t + (off0 + (8 + 2 * (p >> 1) + (p & 1)) * 1024));
+        q.sc = *(const u32x2*)(t + (off0 + 12 * 1024 + 8 * (p >> 1)));  // bytes 2s + (p & 1) are the quarter's
+        q.d = *(const uint16_t*)(d + (uint32_t)(2 * (lane & 15)));
+    } else if constexpr (QT == PGMOE_F16) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) q.c[i] = ldq(t + (offp + (i & ~3) * 1024) + (i & 3) * 1024);
+    } else {
+        q.c0 = ldq(t + offp);
+        q.c1 = ldq(t + offp + 1024);
+        q.c2 = ldq(t + offp + 2048);
+        q.c3 = ldq(t + offp + 3072);
+        q.d = *(const uint32_t*)(t + (off0 + 16 * 1024 + 4 * p));
+    }
+}
+
+struct ThinArgs {
+    const uint8_t *w0, *w1;      // gate / up, or the one matrix
+    int64_t stride0, stride1;    // between experts
+    int N, K;
+    const uint16_t* act;         // fp16 rows: tokens (gather through perm) or pair rows
+    int gather, topk;            // gather: row of pair p is perm[p] / topk, else p
+    int E, P;                    // E = 0: one matrix, pairs 0 .. P - 1 in order
+    const int32_t *offsets, *perm, *tile_off;
+    const float *rs, *topk_w;    // row scale and pair weight (null: 1)
+    const float* bias;           // per output column (null: none)
+    void* out;                   // fp32 rows [P][N] (fp16 with out_f16)
+    int out_f16, act_kind;
+    int kper;                    // super-blocks a split
+    float* raw;                  // split K: raw sums [split][P][NC]
+};
+
+// A finite fp32 value as three bf16 pieces that add up to it, then a zero.
+__device__ __forceinline__ u32x2 thin_split3(float v) {
+    const uint32_t a = __builtin_bit_cast(uint32_t, v) & 0xffff0000u;
+    const float r = v - __builtin_bit_cast(float, a);
+    const uint32_t b = __builtin_bit_cast(uint32_t, r) & 0xffff0000u;
+    const uint32_t c = __builtin_bit_cast(uint32_t, r - __builtin_bit_cast(float, b));
+    return u32x2{(a >> 16) | b, c >> 16};
+}
+
+// Stage shape of a tile of NT token tiles: SPB super-blocks, a row 512 SPB + 16 bytes, so that
+// the 16 rows of a fragment read fall on 16 bank groups.
+template <int NT>
+struct ThinStage {
+    static constexpr int SPB = 4 / NT, ROW = 512 * SPB + 16, PIECES = 32 * SPB;  // 16-byte pieces a row
+    static constexpr int SUMS = 64 * SPB + 16;  // bytes a row: 8 of each 32-element sub-block (thin_split3)
+    static_assert(16 * NT * ROW <= kThinStage && 16 * NT * SUMS <= kThinSums, "a stage fits its buffers");
+};
+
+// One super-block of the wave's R row tiles over NT token tiles; load(r, b) requests row tile
+// r's super-block b (R = 1: the next one before this one's products, else after them).  D of
+// a product: lane l holds weight row l % 16 of tokens 4 (l / 16) + 0..3, so a row's scale is
+// in the lanes that decoded it.
+template <int QT, int R, int NT, bool LOAD, class Load>
+__device__ __forceinline__ void thin_block(const ThinConst& kc, const uint8_t* x, const uint8_t* xs, tf4 (&acc)[R][NT],
+                                           Qtr<QT> (&q)[R], Load& load, int b) {
+    constexpr int T = 16 * ThinStage<NT>::ROW;
+    using W = ThinW<QT>;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const W w(kc, q[r]);
+        if constexpr (LOAD && (R == 1 || NT == 1)) load(r, b + 1);
+        tf4 sum[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) sum[t] = W::POST ? tf4{0.f, 0.f, 0.f, 0.f} : acc[r][t];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            th8 lo, hi, xl[NT], xh[NT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) xl[t] = *(const th8*)(x + T * t + 2 * W::elem(i, 0));
+            if constexpr (NT * R <= 2) {
+#pragma unroll
+                for (int t = 0; t < NT; ++t) xh[t] = *(const th8*)(x + T * t + 2 * W::elem(i, 1));
+            }
+            w.pair(kc, i, lo, hi);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) sum[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[t], lo, sum[t], 0, 0, 0);
+            if constexpr (NT * R > 2) {
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int t = 0; t < NT; ++t) xh[t] = *(const th8*)(x + T * t + 2 * W::elem(i, 1));
+            }
+#pragma unroll
+            for (int t = 0; t < NT; ++t) sum[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[t], hi, sum[t], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (LOAD && R > 1 && NT > 1) load(r, b + 1);
+        if constexpr (W::POST) {
+            const float d = w.scale();
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[r][t][v] = __builtin_fmaf(d, sum[t][v], acc[r][t][v]);
+        } else {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[r][t] = sum[t];
+        }
+        if constexpr (W::MINS) {
+            const tb8 mv = w.mins();
+            const float dm = -w.min_scale();
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+                sum[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const tb8*)(xs + 16 * ThinStage<NT>::SUMS * t), mv,
+                                                                 tf4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[r][t][v] = __builtin_fmaf(dm, sum[t][v], acc[r][t][v]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+
+// A wave's part of a tile of n <= 16 NT pairs from m0: the K loop and the epilogue (a whole
+// copy a token-tile count, so that one's registers never meet another's).  smem: two stages
+// of rows, then two of sums.
+template <int QT, bool GATEUP, int R, int NT, class Load>
+__device__ __forceinline__ void thin_tile(const ThinArgs& A, uint8_t* smem, const uint32_t* rowsrc, const float* rowscale,
+                                          const ThinConst& kc, int m0, int n, int row0, int b0, int nsb,
+                                          Qtr<QT> (&q)[R], Load& load) {
+    using S = ThinStage<NT>;
+    using W = ThinW<QT>;
+    constexpr int CP = 16 * NT * S::PIECES / kThinThreads / S::SPB;  // 16-byte copies a thread and super-block step
+    constexpr int RP = kThinThreads / S::PIECES;                      // rows a copy of the block covers
+    const int tid = threadIdx.x, lane = tid & 63, p = lane >> 4;
+    // The next stage's pieces move a few at a time, beside each super-block of this one: copy
+    // c of step k is 16 bytes of row RP (CP k + c) + tid / PIECES.
+    // The thread's place is formed anew at each step (opaque): held across the loop it costs
+    // registers, and a spilled one a reload that waits for every weight load in flight.
+    auto place = [&](int& pc, int& pr0) {
+        int t = tid;
+        asm volatile("" : "+v"(t));
+        pc = t % S::PIECES, pr0 = t / S::PIECES;
+    };
+    auto fetch = [&](int s, int k, u32x4(&buf)[CP]) {
+        int pc, pr0;
+        place(pc, pr0);
+#pragma unroll
+        for (int c = 0; c < CP; ++c) {  // rows past n repeat row n - 1 (rowsrc), pieces past the split its last
+            const int at = min(32 * S::SPB * s + pc, 32 * nsb - 1);
+            buf[c] = *(const u32x4*)(A.act + (rowsrc[RP * (CP * k + c) + pr0] + (uint32_t)(256 * b0 + 8 * at)));
+        }
+    };
+    auto put = [&](int s, int k, const u32x4(&buf)[CP]) {
+        int pc, pr0;
+        place(pc, pr0);
+#pragma unroll
+        for (int c = 0; c < CP; ++c) {
+            const int r = RP * (CP * k + c) + pr0;
+            if constexpr (W::MINS) {  // four lanes hold a sub-block's 32 elements (whole waves: xor_lane)
+                const th8 h = __builtin_bit_cast(th8, buf[c]);
+                float v = (((float)h[0] + (float)h[1]) + ((float)h[2] + (float)h[3])) +
+                          (((float)h[4] + (float)h[5]) + ((float)h[6] + (float)h[7]));
+                v += xor_lane<1>(v);
+                v += xor_lane<2>(v);
+                if ((tid & 3) == 0)
+                    *(u32x2*)(smem + 2 * kThinStage + (s & 1) * kThinSums + r * S::SUMS + 2 * pc) = thin_split3(v);
+            }
+            *(u32x4*)(smem + (s & 1) * kThinStage + r * S::ROW + 16 * pc) = thin_permute<QT>(buf[c]);
+        }
+    };
+    tf4 acc[R][NT];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[r][t] = tf4{0.f, 0.f, 0.f, 0.f};
+
+    // The last super-block is apart, so that every load of the loop is unconditional (with a
+    // conditional one the compiler waits for every load in flight, not for the oldest).
+    auto reads = [&](int s, const uint8_t*& x, const uint8_t*& xs) {  // the lane's place in stage s
+        int l = lane;
+        asm volatile("" : "+v"(l));
+        x = smem + (s & 1) * kThinStage + (l & 15) * S::ROW + 2 * W::base(l >> 4);
+        xs = smem + 2 * kThinStage + (s & 1) * kThinSums + (l & 15) * S::SUMS + 16 * (l >> 4);
+    };
+    const int stages = (nsb + S::SPB - 1) / S::SPB;
+    {
+        u32x4 first[S::SPB][CP];
+#pragma unroll
+        for (int k = 0; k < S::SPB; ++k) fetch(0, k, first[k]);
+#pragma unroll
+        for (int k = 0; k < S::SPB; ++k) put(0, k, first[k]);
+    }
+    __syncthreads();
+    int b = 0;
+    for (int s = 0; s < stages - 1; ++s) {
+        const uint8_t *x, *xs;
+        reads(s, x, xs);
+#pragma unroll 1
+        for (int k = 0; k < S::SPB; ++k, ++b, x += 512, xs += 64) {
+            u32x4 buf[CP];
+            fetch(s + 1, k, buf);
+            thin_block<QT, R, NT, true>(kc, x, xs, acc, q, load, b);
+            put(s + 1, k, buf);  // buffer (s + 1) & 1: its readers passed the barrier that ended stage s - 1
+        }
+        __syncthreads();
+    }
+    if (row0 >= A.N) return;
+    const uint8_t *x, *xs;
+    reads(stages - 1, x, xs);
+    for (; b < nsb - 1; ++b, x += 512, xs += 64) thin_block<QT, R, NT, true>(kc, x, xs, acc, q, load, b);
+    thin_block<QT, R, NT, false>(kc, x, xs, acc, q, load, b);
+
+    // lane l: output column row0 (+ 16 r) + l % 16 of tokens 16 t + 4 (l / 16) + 0..3
+    const int col = row0 + (lane & 15);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int tok = 16 * t + 4 * p + v;
+            if (tok >= n) continue;
+            const int64_t pr = m0 + tok;
+            if (A.raw) {
+                const int NC = GATEUP ? 2 * A.N : A.N;
+                float* rb = A.raw + ((int64_t)blockIdx.z * A.P + pr) * NC + col;
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    if (col + (GATEUP ? 0 : 16 * r) < A.N) rb[GATEUP ? r * A.N : 16 * r] = acc[r][t][v];
+            } else if constexpr (GATEUP) {
+                if (col < A.N) ((float*)A.out)[pr * A.N + col] = thin_act(A.act_kind, acc[0][t][v]) * acc[1][t][v];
+            } else {
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const int c = col + 16 * r;
+                    if (c >= A.N) continue;
+                    float o = acc[r][t][v] * rowscale[tok];
+                    if (A.bias) o += A.bias[c];
+                    if (A.out_f16)
+                        ((_Float16*)A.out)[pr * A.N + c] = (_Float16)o;
+                    else
+                        ((float*)A.out)[pr * A.N + c] = o;
+                }
+            }
+        }
+}
+
+// Tiles of up to 16 MAXNT pairs; R row tiles a wave (gate/up: gate and up rows).
+template <int QT, bool GATEUP, int R, int MAXNT>
+__global__ __launch_bounds__(kThinThreads, 4) void thin_kernel(const ThinArgs A) {
+    constexpr int ROWS = 16 * MAXNT;
+    static_assert(!GATEUP || R == 2, "gate/up: a gate and an up row tile a wave");
+    __shared__ __attribute__((aligned(16))) uint8_t smem[2 * kThinStage + 2 * kThinSums];
+    __shared__ uint32_t rowsrc[ROWS];  // first element of the tile's activation rows
+    __shared__ float rowscale[ROWS];  // down: rs[p] * topk_w[perm[p]]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tile = blockIdx.y;
+    // the tile's expert: every wave compares the tile with 64 experts' tile ranges at a time
+    int e = 0, m0, n;
+    if (A.E) {
+        if (tile >= A.tile_off[A.E]) return;
+        int first = 0;
+        for (int e0 = 0; e0 < A.E; e0 += 64) {
+            const int ee = min(e0 + lane, A.E - 1);
+            const int lo = A.tile_off[ee], hi = A.tile_off[ee + 1];
+            const uint64_t hit = __ballot(e0 + lane < A.E && lo <= tile && tile < hi);
+            if (hit) {
+                const int l = __builtin_ctzll(hit);
+                e = e0 + l;
+                first = __builtin_amdgcn_readlane(lo, l);
+                break;
+            }
+        }
+        e = __builtin_amdgcn_readfirstlane(e);
+        const int o0 = A.offsets[e], o1 = A.offsets[e + 1];
+        m0 = o0 + (tile - first) * ROWS;
+        n = min(ROWS, o1 - m0);
+    } else {
+        m0 = tile * ROWS;
+        n = min(ROWS, A.P - m0);
+    }
+    const int nb = A.K >> 8;
+    const int b0 = (int)blockIdx.z * A.kper;
+    const int nsb = min(nb - b0, A.kper);
+
+    // the wave's row tiles, and their first super-block on its way
+    const int row0 = ((int)blockIdx.x * kThinWaves + wave) * (GATEUP ? 16 : 16 * R);
+    const int p = lane >> 4;
+    const int ngr = row_groups(A.N);
+    const uint8_t *tb[R], *db[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint8_t* mat = GATEUP && r ? A.w1 + (int64_t)e * A.stride1 : A.w0 + (int64_t)e * A.stride0;
+        const int row = min(GATEUP ? row0 : row0 + 16 * r, 64 * ngr - 16);
+        const int64_t g = (int64_t)(row >> 6) * nb + b0;
+        tb[r] = mat + g * (Tile<QT>::CH * 1024) + (row & 63) * 16;
+        db[r] = mat + (int64_t)ngr * nb * (Tile<QT>::CH * 1024) + (g * 64 + (row & 63)) * 2;
+    }
+    Qtr<QT> q[R];
+    const ThinConst kc = thin_const<QT>(p);
+    uint32_t off0, offp;
+    thin_offsets<QT>(lane, p, off0, offp);
+    auto load = [&](int r, int b) {  // super-block b < nsb of the split
+        thin_load<QT>(q[r], tb[r] + (uint32_t)b * (Tile<QT>::CH * 1024), db[r] + b * 128, off0, offp, lane, p);
+    };
+#pragma unroll
+    for (int r = 0; r < R; ++r) load(r, 0);
+    if (tid < ROWS) {
+        const int pr = m0 + min(tid, n - 1), f = A.perm ? A.perm[pr] : pr;
+        rowsrc[tid] = (uint32_t)(A.gather ? f / A.topk : pr) * (uint32_t)A.K;
+        if (!GATEUP) rowscale[tid] = A.rs ? (A.topk_w ? A.rs[pr] * A.topk_w[f] : A.rs[pr]) : 1.0f;
+    }
+    __syncthreads();
+
+    const int nt = (n + 15) >> 4;
+    if (nt == 1) thin_tile<QT, GATEUP, R, 1>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load);
+    else if (nt == 2) thin_tile<QT, GATEUP, R, 2>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load);
+    else if constexpr (MAXNT > 2) thin_tile<QT, GATEUP, R, 4>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load);
+}
+
+// ---------------------------------------------------------------- when, and launches
+// Tiles of thin_tile_rows() pairs.  A linear of 33 .. 128 rows takes 64, so that its weights
+// are read once or twice less (2048 x 151936 Q6_K, 48 rows: 89 -> 72 us; below and above, 32 and
+// 64 measured alike); the grouped products always 32: gate/up holds two row tiles a wave,
+// and 64 pairs then leave one block a CU (Qwen3 skewed, 301 tokens: 142 us with 32, 154 with 64).
+constexpr int kThinTile = 32;
+int thin_tile_rows() { return kThinTile; }
+
+// Whether the product of P pairs with E matrices [N, K] takes thin tiles.  Each tile decodes
+// its weights again, so the 256-row tiles win once an expert's pairs fill a few of them:
+//   grouped: up to 40 pairs an expert (Qwen3 shape, whole layer: 512 tokens = 32 an expert 206
+//     -> 188 us, 768 = 48 225 -> 235; Mixtral 128 = 32 351 -> 296, 256 = 64 406 -> 447), up to
+//     24 where the 256-row tiles read no scale plane either (Q8_0, F16; Qwen2 shape: 20 an
+//     expert 600 -> 559, 31 657 -> 695);
+//   one matrix, by the weights decoded in all (work): up to 850 M for 256 rows, where the
+//     256-row tiles have one M tile (H = 4096, I = 12288 FFN: 256 rows 162 -> 152 us; Qwen2's
+//     shared expert, 250 rows and 1174 M: 686 -> 705), above that up to 450 M while those tiles
+//     leave most CUs idle (4096 x 6144 Q4_K linear, 512 rows: 77 -> 53; the FFN's down product,
+//     384 rows and 604 M, loses 13 us); fp16 weights, which take the 256-row tiles without any
+//     decode, one tile (I = 5632 FFN: 32 rows 42 -> 36 us, 64 rows 46 -> 49).
+bool thin_takes(int qtype, int64_t P, int E, int N, int K, bool gateup) {
+    if (N % 4 || P * K >= ((int64_t)1 << 31)) return false;  // split sums of four; 32-bit row offsets
+    if (E > 1) return P <= (int64_t)E * (qtype == PGMOE_Q8_0 || qtype == PGMOE_F16 ? 24 : 40);
+    if (qtype == PGMOE_F16) return P <= kThinTile;
+    const int64_t work = (int64_t)div_up(P, kThinTile) * N * K * (gateup ? 2 : 1);
+    return P <= 256 ? work <= 850000000 : work <= 450000000 && (int64_t)div_up(P, 256) * div_up(N, gateup ? 128 : 256) <= 96;
+}
+
+// Splits of K, cut at super-block boundaries: the count with the least estimated time, rounds
+// of two blocks a CU at 3 us a super-block step of a full round (gate/up; one row tile a
+// wave: 1.5) plus the raw sums' way to memory and back at 5 TB/s; no more splits than the
+// 256-row tiles would take for the same product, whose scratch they use.  (H = 4096, I = 12288
+// FFN of 20 rows: 96 gate/up blocks unsplit, 288 in three.)
+static GemmSplit thin_split(const ThinArgs& a, bool gateup, int tile, bool scratch) {
+    const int nb = a.K >> 8;
+    GemmSplit best{1, nb};
+    if (!scratch) return best;
+    const int64_t tiles = div_up(a.P, tile) + (a.E > 0 ? std::min(a.P, a.E) / 2 : 0);
+    const int64_t blocks = tiles * div_up(a.N, 16 * kThinWaves);
+    const int most = gemm_split(a.P, std::max(a.E, 1), a.N, a.K, gateup).ksplit;
+    double t = 1e30;
+    for (int s = 1; s <= most; ++s) {
+        const int kper = div_up(nb, s), n = div_up(nb, kper);
+        const double raw = n > 1 ? (double)n * a.P * a.N * (gateup ? 16 : 8) / 5e6 + 2.0 : 0.0;
+        const double est = (double)div_up(blocks * n, 512) * kper * (gateup ? 3.0 : 1.5) + raw;
+        if (est < t) t = est, best = GemmSplit{n, kper};
+    }
+    return best;
+}
+
+template <int QT>
+static void thin_launch_q(const ThinArgs& a, bool gateup, int tile, const dim3& grid, hipStream_t st) {
+    if (gateup)
+        PG_LAUNCH((thin_kernel<QT, true, 2, 2>), grid, dim3(kThinThreads), 0, st, a);
+    else if (tile == 32)
+        PG_LAUNCH((thin_kernel<QT, false, 1, 2>), grid, dim3(kThinThreads), 0, st, a);
+    else
+        PG_LAUNCH((thin_kernel<QT, false, 1, 4>), grid, dim3(kThinThreads), 0, st, a);
+}
+
+static int thin_launch(const Mats& m, ThinArgs& a, bool gateup, int tile, float* raw, GemmSplit* split,
+                       hipStream_t st) {
+    const GemmSplit sp = thin_split(a, gateup, tile, raw != nullptr);
+    *split = sp;
+    a.kper = sp.kper;
+    a.raw = sp.ksplit > 1 ? raw : nullptr;
+    const int tiles = a.E > 0 ? a.P / tile + std::min(a.P, a.E) : div_up(a.P, tile);
+    const dim3 grid(div_up(a.N, 16 * kThinWaves), tiles, sp.ksplit);
+    switch (m.qtype) {
+    case PGMOE_Q4_1: thin_launch_q<PGMOE_Q4_1>(a, gateup, tile, grid, st); break;
+    case PGMOE_Q4_K: thin_launch_q<PGMOE_Q4_K>(a, gateup, tile, grid, st); break;
+    case PGMOE_Q5_K: thin_launch_q<PGMOE_Q5_K>(a, gateup, tile, grid, st); break;
+    case PGMOE_Q6_K: thin_launch_q<PGMOE_Q6_K>(a, gateup, tile, grid, st); break;
+    case PGMOE_Q8_0: thin_launch_q<PGMOE_Q8_0>(a, gateup, tile, grid, st); break;
+    case PGMOE_F16: thin_launch_q<PGMOE_F16>(a, gateup, tile, grid, st); break;
+    default: return fail(PGMOE_E_UNSUPPORTED, "thin product: qtype %d", m.qtype);
+    }
+    return check_launch(gateup ? "thin gate/up" : "thin down");
+}
+
+// (The scale planes the 256-row tiles read stay required, so that whether a call is accepted
+// does not depend on its size.)
+static bool needs_plane(const Mats& m) { return m.qtype != PGMOE_Q8_0 && m.qtype != PGMOE_F16; }
+
+int launch_thin_gateup(const Mats& g, const Mats& u, const uint16_t* x, int M, int topk, const int32_t* offsets,
+                       const int32_t* perm, const int32_t* tile_off, float* inter, hipStream_t st, float* raw,
+                       int act) {
+    if (needs_plane(g) && (!g.scales || !u.scales))
+        return fail(PGMOE_E_INVALID, "gemm gate/up: K-quant weights need their scale plane (pgmoe_build_scale_plane)");
+    ThinArgs a{};
+    a.w0 = g.base, a.w1 = u.base, a.stride0 = g.stride, a.stride1 = u.stride, a.N = g.N, a.K = g.K;
+    a.act = x, a.gather = perm != nullptr, a.topk = topk;
+    a.E = offsets ? g.n_mats : 0, a.P = M * topk, a.offsets = offsets, a.perm = perm, a.tile_off = tile_off;
+    a.out = inter, a.act_kind = act;
+    GemmSplit sp;
+    int rc = thin_launch(g, a, true, kThinTile, raw, &sp, st);
+    if (rc || sp.ksplit == 1) return rc;
+    return launch_split_reduce(1, raw, sp.ksplit, a.P, g.N, nullptr, nullptr, nullptr, inter, st, act);
+}
+
+int launch_thin_down(const Mats& d, const uint16_t* a16, const float* rs, int M, int topk, const int32_t* offsets,
+                     const int32_t* perm, const int32_t* tile_off, const float* topk_w, float* partial,
+                     hipStream_t st, float* raw) {
+    if (needs_plane(d) && !d.scales)
+        return fail(PGMOE_E_INVALID, "gemm down: K-quant weights need their scale plane (pgmoe_build_scale_plane)");
+    ThinArgs a{};
+    a.w0 = d.base, a.stride0 = d.stride, a.N = d.N, a.K = d.K, a.act = a16, a.topk = topk;
+    a.E = offsets ? d.n_mats : 0, a.P = M * topk, a.offsets = offsets, a.perm = perm, a.tile_off = tile_off;
+    a.rs = rs, a.topk_w = topk_w, a.out = partial;
+    GemmSplit sp;
+    int rc = thin_launch(d, a, false, kThinTile, raw, &sp, st);
+    if (rc || sp.ksplit == 1) return rc;
+    return launch_split_reduce(0, raw, sp.ksplit, a.P, d.N, rs, topk_w, perm, partial, st, PGMOE_ACT_SILU);
+}
+
+int launch_thin_linear(const Mats& w, const uint16_t* x, int M, const float* bias, void* out, int out_f16, float* raw,
+                       hipStream_t st) {
+    ThinArgs a{};
+    a.w0 = w.base, a.N = w.N, a.K = w.K, a.act = x, a.topk = 1, a.P = M;
+    a.bias = bias, a.out = out, a.out_f16 = out_f16;
+    GemmSplit sp;
+    int rc = thin_launch(w, a, false, M > 32 && M <= 128 ? 64 : 32, raw, &sp, st);
+    if (rc || sp.ksplit == 1) return rc;
+    return launch_split_reduce(2, raw, sp.ksplit, M, w.N, bias, nullptr, nullptr, out, st, out_f16);
+}
+
+}  // namespace pgmoe

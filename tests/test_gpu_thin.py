@@ -1,0 +1,105 @@
+"""GPU parity of the thin tiles (csrc/thin.hip): products of few rows an expert.
+
+Linears, MoE layers and dense FFNs at the edges of the tiles (16 tokens an MFMA, 32 or 64 rows
+a tile, stages of 4, 2 and 1 super-blocks, row tiles past the last row) and of the rule that
+chooses them, in every device format, against float64 products on the oracle's weights.
+
+A linear's bound: fp16 rounding of each weight (2^-11 of it at most; the K-quants' integer
+codes are exact) and fp32 sums of K products, so |d| <= 2^-11 sum |x w| + K 2^-23 sum |x| (|w| +
+offset part); the second term is held at 2^-13 sum |x w| with room for the offset part.
+"""
+
+import numpy as np
+import pytest
+
+import oracle
+from gpu_helpers import build_pair, check_forward_routing, check_layer_output, log
+from pgmoe.synth import DenseSpec, LayerSpec, SyntheticDense, random_blocks
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+F16, Q4_1, Q8_0, Q4_K, Q5_K, Q6_K = 1, 3, 8, 12, 13, 14
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    yield
+    torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("qt", [Q4_1, Q8_0, Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("N,K,xs", [(68, 256, 1.0), (260, 1280, 1.0), (1540, 768, 1.0), (132, 2304, 3e4)])
+def test_linear_tiles(qt, N, K, xs):
+    from pgmoe import GGUFQuantLinear
+    dev = torch.device("cuda", 0)
+    rng = np.random.default_rng(N + K + qt)
+    raw = random_blocks(rng, qt, N, K, 0.01)
+    bias = torch.from_numpy(rng.standard_normal(N).astype(np.float32))
+    lin = GGUFQuantLinear("w8", K, N, qt, raw=raw, bias=bias, device=dev)
+    w = oracle.dequant(qt, raw, N, K).astype(np.float64)
+    x = (np.clip(rng.standard_normal((300, K)), -2, 2) * xs).astype(np.float16)
+    ref = x.astype(np.float64) @ w.T + bias.numpy()
+    bound = (2.0 ** -11 + 2.0 ** -13) * (np.abs(x.astype(np.float64)) @ np.abs(w).T) + 1e-5
+    for M in (9, 16, 17, 32, 33, 48, 64, 65, 96, 128, 129, 300):
+        log(f"thin linear qt={qt} N={N} K={K} x*{xs} M={M}")
+        xm = torch.from_numpy(x[:M]).to(dev)
+        got = lin(xm.float()).cpu().numpy()
+        assert np.all(np.abs(got - ref[:M]) <= bound[:M]), f"M={M}: {np.max(np.abs(got - ref[:M]) / bound[:M]):.2f}"
+        if xs == 1.0:  # fp16 output: the fp32 result rounded
+            assert np.array_equal(lin(xm).cpu().numpy(), got.astype(np.float16))
+
+
+@pytest.mark.parametrize("gate_up,down", [(Q4_K, Q6_K), (Q5_K, Q4_K), (Q6_K, Q5_K), (Q8_0, Q8_0), (Q4_1, Q4_1),
+                                          (F16, F16)])
+def test_layer_tiles(gate_up, down):
+    """A skewed router: with M tokens the first expert holds about M pairs (tiles of 32 and a
+    remainder), the others few or none; M = 160 / 161 lie on both sides of 40 pairs an expert."""
+    spec = LayerSpec("thin", 768, 8, 2, 512, (gate_up, gate_up, down), shared_inter=256,
+                     shared_qtypes=(gate_up, gate_up, down), shared_gate=True)
+    # float weights at their own scale: at 0.01 (2e-4) the SwiGLU rows, near 1e-6, fall among
+    # fp16's subnormals (spacing 6e-8), and their fp16 form alone is off by up to 3e-2 a value
+    lay, ol, mod = build_pair(spec, seed=5, scale=1.0 if gate_up == F16 else 0.01)
+    bias = np.array([6, 1, 0, 0, -1, -1, -2, -8], np.float32)
+    mod.set_router_bias(torch.from_numpy(bias))
+    ol = oracle.OracleLayer.from_gguf(lay.gguf, lay.config, router_bias=bias)
+    for M in (9, 16, 33, 47, 96, 97, 160, 161):
+        log(f"thin layer {gate_up}/{down} M={M}")
+        x = lay.draw_x(M)
+        got = mod(torch.from_numpy(x).to("cuda:0")).cpu().numpy()
+        _, idx, w = ol.route(x)
+        check_forward_routing(mod, M, idx, w)
+        check_layer_output(got, ol.forward_tokens(x, idx, w))
+
+
+def test_dense_sides_of_the_rule_and_replays():
+    """Both products on thin tiles, only the down one, and neither; a captured forward on thin
+    tiles equals the eager one at every replay."""
+    from pgmoe import HipDenseMLP
+    dev = torch.device("cuda", 0)
+    lay = SyntheticDense(DenseSpec("thin", 1024, 25600, (Q4_K, Q4_K, Q6_K)), seed=2, scale=0.01)
+    mod = HipDenseMLP(lay.gguf, lay.config, 0, dev)
+    mats = [(t.qtype, *t.shape, lay.tensor(f"ffn_{p}.weight")) for p in ("gate", "up", "down")
+            for t in [lay.gguf.tensors[f"blk.0.ffn_{p}.weight"]]]
+    for M in (9, 100, 256, 257, 600):
+        log(f"thin dense M={M}")
+        x = lay.draw_x(M)
+        toks = np.unique(np.linspace(0, M - 1, 5).astype(np.int64))
+        got = mod(torch.from_numpy(x).to(dev)).cpu().numpy()
+        check_layer_output(got[toks], oracle.dense_forward(x, *mats, tokens=toks))
+    x = torch.from_numpy(lay.draw_x(40)).to(dev)
+    side = torch.cuda.Stream(dev)
+    side.wait_stream(torch.cuda.current_stream(dev))
+    with torch.cuda.stream(side):
+        mod(x)
+    side.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        out = mod(x)
+    for seed in range(3):
+        x.copy_(torch.randn(x.shape, generator=torch.Generator().manual_seed(seed)).to(torch.float16))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, mod(x))
