@@ -1,5 +1,7 @@
 // R1 + R2: router logits in a fixed reduction order, then softmax / top-k / renorm.
 // Reference: pygguf_engine/model.py:902-907.
+#include <algorithm>
+
 #include "common.h"
 #include "launch.h"
 
@@ -219,6 +221,116 @@ __global__ __launch_bounds__(256) void topk_kernel(const float* __restrict__ log
     }
 }
 
+// ---------------------------------------------------------------- matrix-core router
+// The same logits on v_mfma_f32_16x16x4_f32, whose every output element is one chain of fused
+// multiply-adds over ascending k, each rounded as fmaf rounds (checked bit for bit), so a
+// slot's chain is a run of MFMAs.  A block of 16 waves owns 16 experts and walks tiles of 16
+// tokens: wave (g, h) does the slots 8g + 4h .. + 3 (32 contiguous elements of every 512) of
+// the tile, holding its share of the expert rows in registers, and the 64 slot sums of each
+// logit meet in the xor tree (32, 16, ..., 1) through LDS.  Lane (row r, p) loads the chunk of
+// slot 8g + 4h + p; two lane exchanges transpose the four lanes' chunks into the operands
+// (elements p and p + 4 of each).  J = H / 512 chunks a slot.
+// Each tile's 2 us of matrix work, its LDS tree and the barriers between them follow one another
+// (one block a CU); the first tile waits for 192 KB of rows.  Measured with its top-k, before
+// (LDS-tiled or wave-tile FMAs) -> now: H = 2048, 128 experts, 301 / 512 / 1024 / 4096 tokens 19.4 ->
+// 15.0, 21.8 -> 15.1, 37.3 -> 19.2, 50.6 -> 40.5 us; H = 3584, 64 experts, 1024 / 2048 tokens 25.8 ->
+// 20.7, 45.3 -> 26.4.  Two 1024-thread blocks a CU (64 registers) and a wave a tile (with the
+// tree in registers; 33 us for any token count) measured slower.
+typedef float rf4 __attribute__((ext_vector_type(4)));
+
+// r[k] of lane group p becomes V[k][p] where it was V[p][k] (p = lane / 16, 4 x 4).
+__device__ __forceinline__ void transpose4(uint32_t (&r)[4]) {
+    auto a = __builtin_amdgcn_permlane32_swap(r[0], r[2], false, false);
+    auto b = __builtin_amdgcn_permlane32_swap(r[1], r[3], false, false);
+    auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+    auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+    r[0] = c[0], r[1] = c[1], r[2] = d[0], r[3] = d[1];
+}
+
+constexpr int kRmThreads = 1024;
+template <int J>
+__global__ __launch_bounds__(kRmThreads) void router_mfma_kernel(const uint16_t* __restrict__ x,
+                                                                 const float* __restrict__ W,
+                                                                 const float* __restrict__ bias, int M, int E,
+                                                                 float* __restrict__ logits) {
+    constexpr int H = 512 * J;
+    __shared__ rf4 part[64][64];      // slot sums [slot][lane of the tile's D layout]
+    __shared__ float quarter[4][256];
+    const int tid = threadIdx.x, lane = tid & 63, p = lane >> 4, r = lane & 15;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int e0 = 16 * (int)blockIdx.y, lo = 32 * w + 8 * p;  // 64 g + 32 h = 32 w
+    uint32_t wt[J][2][4];
+    {
+        const float* wr = W + (int64_t)min(e0 + r, E - 1) * H + lo;
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                const float4 f = *(const float4*)(wr + 512 * j + 4 * m);
+                wt[j][m][0] = __builtin_bit_cast(uint32_t, f.x), wt[j][m][1] = __builtin_bit_cast(uint32_t, f.y);
+                wt[j][m][2] = __builtin_bit_cast(uint32_t, f.z), wt[j][m][3] = __builtin_bit_cast(uint32_t, f.w);
+            }
+    }
+    uint4 xb[J];
+    auto load = [&](int j, int m0) {  // (rows past M repeat the last: never stored)
+        xb[j] = *(const uint4*)(x + (int64_t)min(m0 + r, M - 1) * H + lo + 512 * j);
+    };
+    int m0 = 16 * (int)blockIdx.x;
+#pragma unroll
+    for (int j = 0; j < J; ++j) load(j, m0);
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) transpose4(wt[j][m]);
+    for (; m0 < M; m0 += 16 * (int)gridDim.x) {
+        const int next = m0 + 16 * (int)gridDim.x;
+        rf4 sum[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sum[q] = rf4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            const uint4 v = xb[j];
+            uint32_t xt[4];  // (element k, element k + 4) pairs of the chunk's halves
+            xt[0] = __builtin_amdgcn_perm(v.z, v.x, 0x05040100u);
+            xt[1] = __builtin_amdgcn_perm(v.z, v.x, 0x07060302u);
+            xt[2] = __builtin_amdgcn_perm(v.w, v.y, 0x05040100u);
+            xt[3] = __builtin_amdgcn_perm(v.w, v.y, 0x07060302u);
+            load(j, next);  // the next tile's, past the last one a repeat
+            transpose4(xt);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                sum[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(lo_half(xt[q]), __builtin_bit_cast(float, wt[j][0][q]),
+                                                              sum[q], 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                sum[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(hi_half(xt[q]), __builtin_bit_cast(float, wt[j][1][q]),
+                                                              sum[q], 0, 0, 0);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) part[4 * w + q][lane] = sum[q];
+        __syncthreads();
+        // thread (z, token, expert): the tree over the slots of low bits z and z + 4, then the
+        // four z; D element v of lane l is token 4 (l / 16) + v, expert l % 16
+        const int tok = (tid >> 4) & 15, e = tid & 15, z = tid >> 8;
+        const int i = ((tok >> 2) * 16 + e) * 4 + (tok & 3);
+        float s[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            float a[8];
+#pragma unroll
+            for (int g = 0; g < 8; ++g) a[g] = ((const float*)part[8 * g + z + 4 * k])[i];
+            const float b0 = a[0] + a[4], b1 = a[1] + a[5], b2 = a[2] + a[6], b3 = a[3] + a[7];
+            s[k] = (b0 + b2) + (b1 + b3);
+        }
+        quarter[z][tid & 255] = s[0] + s[1];
+        __syncthreads();
+        if (tid < 256 && m0 + tok < M && e0 + e < E) {
+            const float v = (quarter[0][tid] + quarter[2][tid]) + (quarter[1][tid] + quarter[3][tid]);
+            logits[(int64_t)(m0 + tok) * E + e0 + e] = bias ? v + bias[e0 + e] : v;
+        }
+    }
+}
+
 int launch_router_logits(const uint16_t* x, const float* W, const float* bias, int M, int H, int E,
                          float* logits, hipStream_t st, const float* extra_w, float* extra_out, float* xsum) {
     if (M <= 0) return PGMOE_OK;
@@ -241,6 +353,25 @@ int launch_router_logits(const uint16_t* x, const float* W, const float* bias, i
         PG_ROUTER(4, 1);
     else if (M <= 8)
         PG_ROUTER(8, 1);
+    else if (!extra_w && !xsum && E >= 16 && H % 512 == 0 && H <= 4096 && (int64_t)M * E >= 24576) {
+        // the matrix-core form from 24576 logits on (fewer: its 5 us of loads and hand-over in one
+        // round outlast the vector forms; crossovers at 128 x ~170, 64 x ~450, 16 x ~1700 tokens)
+        const int ne = div_up(E, 16), nt = div_up(M, 16);
+        const dim3 grid(std::min(nt, std::max(1, 256 / ne)), ne);  // one block a CU
+#define PG_RM(J) \
+    case J: PG_LAUNCH(router_mfma_kernel<J>, grid, dim3(kRmThreads), 0, st, x, W, bias, M, E, logits); break
+        switch (H >> 9) {
+            PG_RM(1);
+            PG_RM(2);
+            PG_RM(3);
+            PG_RM(4);
+            PG_RM(5);
+            PG_RM(6);
+            PG_RM(7);
+            PG_RM(8);
+        }
+#undef PG_RM
+    }
     else if (!extra_w && !xsum && E >= 16 && H % kRgH == 0 && div_up(M, kRgT) * div_up(E, kRgE) >= 1024) {
         PG_LAUNCH(router_gemm_kernel, dim3(div_up(M, kRgT), div_up(E, kRgE)), dim3(256), 0, st, x, W, bias, M, H, E,
                   logits);

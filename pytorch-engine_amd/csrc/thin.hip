@@ -34,9 +34,6 @@
 
 namespace pgmoe {
 
-#ifndef PG_THIN_R
-#define PG_THIN_R 1
-#endif
 constexpr int kThinRows = 64;  // most pairs a tile
 constexpr int kThinWaves = 8;
 constexpr int kThinThreads = 64 * kThinWaves;
