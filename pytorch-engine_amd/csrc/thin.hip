@@ -678,14 +678,16 @@ int thin_tile_rows() { return kThinTile; }
 //     256-row tiles have one M tile (H = 4096, I = 12288 FFN: 256 rows 162 -> 152 us; Qwen2's
 //     shared expert, 250 rows and 1174 M: 686 -> 705), above that up to 450 M while those tiles
 //     leave most CUs idle (4096 x 6144 Q4_K linear, 512 rows: 77 -> 53; the FFN's down product,
-//     384 rows and 604 M, loses 13 us); fp16 weights, which take the 256-row tiles without any
+//     384 rows and 604 M, loses 13 us; above 512 rows up to 150 M: 2048 x 1024 Q8_0, 1024 rows 35
+//     -> 17, but an I = 5632 down product of 1024 rows and 369 M loses 6); fp16 weights, which take the 256-row tiles without any
 //     decode, one tile (I = 5632 FFN: 32 rows 42 -> 36 us, 64 rows 46 -> 49).
 bool thin_takes(int qtype, int64_t P, int E, int N, int K, bool gateup) {
     if (N % 4 || P * K >= ((int64_t)1 << 31)) return false;  // split sums of four; 32-bit row offsets
     if (E > 1) return P <= (int64_t)E * (qtype == PGMOE_Q8_0 || qtype == PGMOE_F16 ? 24 : 40);
     if (qtype == PGMOE_F16) return P <= kThinTile;
     const int64_t work = (int64_t)div_up(P, kThinTile) * N * K * (gateup ? 2 : 1);
-    return P <= 256 ? work <= 850000000 : work <= 450000000 && (int64_t)div_up(P, 256) * div_up(N, gateup ? 128 : 256) <= 96;
+    if (P <= 256) return work <= 850000000;
+    return work <= (P <= 512 ? 450000000 : 150000000) && (int64_t)div_up(P, 256) * div_up(N, gateup ? 128 : 256) <= 96;
 }
 
 // Splits of K, cut at super-block boundaries: the count with the least estimated time, rounds
