@@ -180,6 +180,10 @@ int launch_thin_down(const Mats& d, const uint16_t* a16, const float* rs, int M,
                      hipStream_t st, float* raw);
 int launch_thin_linear(const Mats& w, const uint16_t* x, int M, const float* bias, void* out, int out_f16, float* raw,
                        hipStream_t st);
+// A decode linear (M <= 8) on a thin tile, where thin_takes_decode: exact weights, fp32 sums.
+bool thin_takes_decode(int qtype, int M, int N, int K);
+int launch_thin_decode(const Mats& w, const uint16_t* x, int M, const float* bias, void* out, int out_f16,
+                       hipStream_t st);
 int64_t layout_bytes(int qtype, int64_t rows, int64_t cols);
 // Scale plane (relayout.hip): bytes of one matrix's plane (0 for Q8_0, -1 if unsupported)
 // and its load-time construction from the device layout.

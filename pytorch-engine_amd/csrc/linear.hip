@@ -4,7 +4,7 @@
 // / exec_w8a16_matmul, :1165-1420), FusedLinearPack.forward_single_concat (:1895-1898) and
 // GGUFQuantLinear.embed_lookup (:1839-1863).
 //   M <= 8 : the decode GEMV in its single-matrix mode (dec_gu_kernel<..., kLinear>), bias
-//            and output rounding in its epilogue;
+//            and output rounding in its epilogue; an output head's 3 .. 8 rows on a thin tile;
 //   M  > 8 : thin tiles (thin.hip; bias and rounding in their epilogue or split reduce) up to
 //            a few hundred rows, else identity dispatch, the grouped MFMA GEMM (the down
 //            product's form, A = x read directly, unit row scales) and a bias / fp16 pass when
@@ -138,6 +138,8 @@ size_t linear_ws_bytes(const Mats& w, int M, bool staged) {
 int launch_linear(const Mats& w, const float* bias, const uint16_t* x, int M, void* out, int out_f16, uint8_t* ws,
                   size_t ws_bytes, hipStream_t st) {
     if (M == 0) return PGMOE_OK;
+    if (linear_gemv(M, w.K) && thin_takes_decode(w.qtype, M, w.N, w.K))
+        return launch_thin_decode(w, x, M, bias, out, out_f16, st);
     if (linear_gemv(M, w.K)) return launch_dec_linear(w, x, M, bias, out, out_f16, st);
     const bool staged = bias || out_f16;
     if (ws_bytes < linear_ws_bytes(w, M, staged))

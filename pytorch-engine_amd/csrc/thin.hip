@@ -199,9 +199,15 @@ template <> struct ThinW<PGMOE_Q6_K> {
         qh[0] = q.qh.x, qh[1] = q.qh.y, qh[2] = q.qh.z, qh[3] = q.qh.w;
     }
     // step pair i: chunk la (i even) or lb, its first or second 8 bytes; sub-blocks s = i & 1
-    // (low nibbles) and s + 2 (high), high bits 2s of each qh byte
+    // (low nibbles) and s + 2 (high), high bits 2s of each qh byte.  EX: what the rounding above
+    // 2048 took away too (-1, 0 or 1: exact), so that lo + rlo and hi + rhi are sc (q - 32).
     __device__ __forceinline__ void pair(const ThinConst& kc, int i, th8& lo, th8& hi) const {
-        th2 m[4], n[4];
+        th8 rlo, rhi;
+        pair<false>(kc, i, lo, hi, rlo, rhi);
+    }
+    template <bool EX>
+    __device__ __forceinline__ void pair(const ThinConst& kc, int i, th8& lo, th8& hi, th8& rlo, th8& rhi) const {
+        th2 m[4], n[4], rm[4], rn[4];
         const int s = i & 1;
         const th2 a = s ? th2{s01.y, s01.y} : th2{s01.x, s01.x}, b = s ? th2{s23.y, s23.y} : th2{s23.x, s23.x};
 #pragma unroll
@@ -213,11 +219,20 @@ template <> struct ThinW<PGMOE_Q6_K> {
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            m[k] = (m[k] - h2(1056.0f)) * a;
-            n[k] = (n[k] - h2(1056.0f)) * b;
+            const th2 cm = m[k] - h2(1056.0f), cn = n[k] - h2(1056.0f);
+            m[k] = cm * a;
+            n[k] = cn * b;
+            if constexpr (EX) {
+                rm[k] = pk_fma(cm, a, -m[k]);
+                rn[k] = pk_fma(cn, b, -n[k]);
+            }
         }
         lo = cat8(m);
         hi = cat8(n);
+        if constexpr (EX) {
+            rlo = cat8(rm);
+            rhi = cat8(rn);
+        }
     }
     __device__ static __forceinline__ constexpr int elem(int i, int half) {
         return 32 * (i & 1) + 8 * (i >> 1) + 64 * half;
@@ -403,7 +418,7 @@ struct ThinStage {
 // r's super-block b (R = 1: the next one before this one's products, else after them).  D of
 // a product: lane l holds weight row l % 16 of tokens 4 (l / 16) + 0..3, so a row's scale is
 // in the lanes that decoded it.
-template <int QT, int R, int NT, bool LOAD, class Load>
+template <int QT, int R, int NT, bool LOAD, bool EX, class Load>
 __device__ __forceinline__ void thin_block(const ThinConst& kc, const uint8_t* x, const uint8_t* xs, tf4 (&acc)[R][NT],
                                            Qtr<QT> (&q)[R], Load& load, int b) {
     constexpr int T = 16 * ThinStage<NT>::ROW;
@@ -424,9 +439,16 @@ __device__ __forceinline__ void thin_block(const ThinConst& kc, const uint8_t* x
 #pragma unroll
                 for (int t = 0; t < NT; ++t) xh[t] = *(const th8*)(x + T * t + 2 * W::elem(i, 1));
             }
-            w.pair(kc, i, lo, hi);
+            th8 rlo, rhi;
+            if constexpr (EX && QT == PGMOE_Q6_K)
+                w.template pair<true>(kc, i, lo, hi, rlo, rhi);
+            else
+                w.pair(kc, i, lo, hi);
 #pragma unroll
             for (int t = 0; t < NT; ++t) sum[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[t], lo, sum[t], 0, 0, 0);
+            if constexpr (EX && QT == PGMOE_Q6_K)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) sum[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[t], rlo, sum[t], 0, 0, 0);
             if constexpr (NT * R > 2) {
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -434,6 +456,9 @@ __device__ __forceinline__ void thin_block(const ThinConst& kc, const uint8_t* x
             }
 #pragma unroll
             for (int t = 0; t < NT; ++t) sum[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[t], hi, sum[t], 0, 0, 0);
+            if constexpr (EX && QT == PGMOE_Q6_K)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) sum[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[t], rhi, sum[t], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (LOAD && R > 1 && NT > 1) load(r, b + 1);
@@ -466,7 +491,7 @@ __device__ __forceinline__ void thin_block(const ThinConst& kc, const uint8_t* x
 // A wave's part of a tile of n <= 16 NT pairs from m0: the K loop and the epilogue (a whole
 // copy a token-tile count, so that one's registers never meet another's).  smem: two stages
 // of rows, then two of sums.
-template <int QT, bool GATEUP, int R, int NT, class Load>
+template <int QT, bool GATEUP, int R, int NT, bool EX, class Load>
 __device__ __forceinline__ void thin_tile(const ThinArgs& A, uint8_t* smem, const uint32_t* rowsrc, const float* rowscale,
                                           const ThinConst& kc, int m0, int n, int row0, int b0, int nsb,
                                           Qtr<QT> (&q)[R], Load& load) {
@@ -542,7 +567,7 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& A, uint8_t* smem, cons
         for (int k = 0; k < S::SPB; ++k, ++b, x += 512, xs += 64) {
             u32x4 buf[CP];
             fetch(s + 1, k, buf);
-            thin_block<QT, R, NT, true>(kc, x, xs, acc, q, load, b);
+            thin_block<QT, R, NT, true, EX>(kc, x, xs, acc, q, load, b);
             put(s + 1, k, buf);  // buffer (s + 1) & 1: its readers passed the barrier that ended stage s - 1
         }
         __syncthreads();
@@ -550,8 +575,8 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& A, uint8_t* smem, cons
     if (row0 >= A.N) return;
     const uint8_t *x, *xs;
     reads(stages - 1, x, xs);
-    for (; b < nsb - 1; ++b, x += 512, xs += 64) thin_block<QT, R, NT, true>(kc, x, xs, acc, q, load, b);
-    thin_block<QT, R, NT, false>(kc, x, xs, acc, q, load, b);
+    for (; b < nsb - 1; ++b, x += 512, xs += 64) thin_block<QT, R, NT, true, EX>(kc, x, xs, acc, q, load, b);
+    thin_block<QT, R, NT, false, EX>(kc, x, xs, acc, q, load, b);
 
     // lane l: output column row0 (+ 16 r) + l % 16 of tokens 16 t + 4 (l / 16) + 0..3
     const int col = row0 + (lane & 15);
@@ -586,7 +611,8 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& A, uint8_t* smem, cons
         }
 }
 
-// Tiles of up to 16 MAXNT pairs; R row tiles a wave (gate/up: gate and up rows).
+// Tiles of up to 16 MAXNT pairs; R row tiles a wave (gate/up: gate and up rows).  MAXNT 1: a
+// decode linear (EX: exact weights).
 template <int QT, bool GATEUP, int R, int MAXNT>
 __global__ __launch_bounds__(kThinThreads, 4) void thin_kernel(const ThinArgs A) {
     constexpr int ROWS = 16 * MAXNT;
@@ -655,9 +681,11 @@ __global__ __launch_bounds__(kThinThreads, 4) void thin_kernel(const ThinArgs A)
     __syncthreads();
 
     const int nt = (n + 15) >> 4;
-    if (nt == 1) thin_tile<QT, GATEUP, R, 1>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load);
-    else if (nt == 2) thin_tile<QT, GATEUP, R, 2>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load);
-    else if constexpr (MAXNT > 2) thin_tile<QT, GATEUP, R, 4>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load);
+    if (MAXNT == 1 || nt == 1) thin_tile<QT, GATEUP, R, 1, MAXNT == 1>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load);
+    else if constexpr (MAXNT > 1) {
+        if (nt == 2) thin_tile<QT, GATEUP, R, 2, false>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load);
+        else if constexpr (MAXNT > 2) thin_tile<QT, GATEUP, R, 4, false>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load);
+    }
 }
 
 // ---------------------------------------------------------------- when, and launches
@@ -775,6 +803,33 @@ int launch_thin_down(const Mats& d, const uint16_t* a16, const float* rs, int M,
     int rc = thin_launch(d, a, false, kThinTile, raw, &sp, st);
     if (rc || sp.ksplit == 1) return rc;
     return launch_split_reduce(0, raw, sp.ksplit, a.P, d.N, rs, topk_w, perm, partial, st, PGMOE_ACT_SILU);
+}
+
+// A decode linear (M <= 8) of K-quants on one thin tile, weights exact (the GEMV's precision:
+// its error against float64 falls from 2e-5 .. 3.5e-6 to 2.5e-7 .. 1.3e-7).  The GEMV decodes a
+// weight once but spends a dot2 and two LDS bytes on it for each token, so 8 tokens cost it twice
+// the weights' time; here 16 rows of MFMA cost what one does.  2048 x 151936, us GEMV -> here:
+// Q6_K 3 rows 70 -> 62, 8 rows 121 -> 64; Q4_K 56 -> 45, 103 -> 46; Q5_K 62 -> 53, 107 -> 55 (two
+// rows: Q6_K 60 -> 62).  Q8_0's d q is no fp16 value, so it stays there.  K is not split, so
+// that outputs depend on no other rows of a pack: from a block a CU on.
+bool thin_takes_decode(int qtype, int M, int N, int K) {
+    return (qtype == PGMOE_Q4_K || qtype == PGMOE_Q5_K || qtype == PGMOE_Q6_K) && M > 2 && N >= 32768 && N % 4 == 0 &&
+           (int64_t)M * K < ((int64_t)1 << 31);
+}
+
+int launch_thin_decode(const Mats& w, const uint16_t* x, int M, const float* bias, void* out, int out_f16,
+                       hipStream_t st) {
+    ThinArgs a{};
+    a.w0 = w.base, a.N = w.N, a.K = w.K, a.act = x, a.topk = 1, a.P = M;
+    a.bias = bias, a.out = out, a.out_f16 = out_f16, a.kper = w.K >> 8;
+    const dim3 grid(div_up(a.N, 16 * kThinWaves), 1, 1);
+    switch (w.qtype) {
+    case PGMOE_Q4_K: PG_LAUNCH((thin_kernel<PGMOE_Q4_K, false, 1, 1>), grid, dim3(kThinThreads), 0, st, a); break;
+    case PGMOE_Q5_K: PG_LAUNCH((thin_kernel<PGMOE_Q5_K, false, 1, 1>), grid, dim3(kThinThreads), 0, st, a); break;
+    case PGMOE_Q6_K: PG_LAUNCH((thin_kernel<PGMOE_Q6_K, false, 1, 1>), grid, dim3(kThinThreads), 0, st, a); break;
+    default: return fail(PGMOE_E_UNSUPPORTED, "thin decode linear: qtype %d", w.qtype);
+    }
+    return check_launch("thin linear");
 }
 
 int launch_thin_linear(const Mats& w, const uint16_t* x, int M, const float* bias, void* out, int out_f16, float* raw,

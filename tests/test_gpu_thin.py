@@ -52,6 +52,30 @@ def test_linear_tiles(qt, N, K, xs):
             assert np.array_equal(lin(xm).cpu().numpy(), got.astype(np.float16))
 
 
+@pytest.mark.parametrize("qt", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("K", [256, 1280, 2304])
+def test_decode_linear_of_many_rows(qt, K):
+    """3 .. 8 tokens of an output head: exact products in fp32 sums of K / 32 + K / 128 terms, each
+    rounded to 2^-24 of a partial sum, at most 90 x 6e-8 = 5.4e-6 of the result's norm (a weight
+    rounded to fp16 would show 1e-4); either side of the rule's tokens and rows agrees."""
+    from pgmoe import GGUFQuantLinear
+    dev = torch.device("cuda", 0)
+    rng = np.random.default_rng(K + qt)
+    N = 32768 + 36
+    raw = random_blocks(rng, qt, N, K, 0.01)
+    bias = torch.from_numpy(rng.standard_normal(N).astype(np.float32))
+    lin = GGUFQuantLinear("w8", K, N, qt, raw=raw, bias=bias, device=dev)
+    w = torch.from_numpy(oracle.dequant(qt, raw, N, K)).to(dev).double()
+    x = torch.from_numpy(rng.standard_normal((9, K)).astype(np.float16)).to(dev)
+    ref = x.double() @ w.T + bias.to(dev).double()
+    for M in (1, 2, 3, 5, 8, 9):
+        log(f"thin decode linear qt={qt} K={K} M={M}")
+        got = lin(x[:M].float())
+        err = float((got.double() - ref[:M]).norm() / ref[:M].norm())
+        assert err <= (5.4e-6 if 3 <= M <= 8 else 1e-3), (M, err)
+        assert torch.equal(lin(x[:M]), got.to(torch.float16))
+
+
 @pytest.mark.parametrize("gate_up,down", [(Q4_K, Q6_K), (Q5_K, Q4_K), (Q6_K, Q5_K), (Q8_0, Q8_0), (Q4_1, Q4_1),
                                           (F16, F16)])
 def test_layer_tiles(gate_up, down):
