@@ -210,11 +210,12 @@ static DenseLayout dense_layout(int M, int I, int H) {
     o.w = take(c, gemm ? (size_t)M * 4 : 0);
     o.inter = take(c, (size_t)M * I * 4);
     o.isum = take(c, gemm ? 0 : (size_t)M * (I / 16) * 4);
-    o.a16 = take(c, gemm ? (size_t)M * I * 2 : 0);
-    o.rs = take(c, gemm ? (size_t)M * 4 : 0);
+    o.a16 = take(c, (size_t)(gemm ? M : 2 * M) * I * 2);  // decode: two rows a token
+    o.rs = take(c, (size_t)M * 4);
     o.raw = take(c, gemm ? std::max(gemm_split_bytes_upto(M, 1, I, H, true), gemm_split_bytes_upto(M, 1, H, I, false))
-                         : 0);
-    o.total = c;
+                         : M > 2 ? thin_dec_raw_bytes(I, H) : 0);
+    // a workspace for many tokens serves fewer
+    o.total = gemm ? std::max(c, dense_layout(decode_tokens_max(), I, H).total) : c;
     return o;
 }
 
@@ -261,6 +262,9 @@ int pgmoe_dense_forward(const pgmoe_dense* D, const uint16_t* x, int32_t M, floa
 #define WS(T, f) reinterpret_cast<T*>(b + o.f)
     const hipStream_t st = as_stream(stream);
     if (M <= decode_tokens_max()) {  // gate/up + SwiGLU, then down straight into out
+        if (thin_takes_dense_decode(g, u, d, M))
+            return launch_thin_dense_decode(g, u, d, x, M, D->act, WS(float, inter), WS(uint16_t, a16), WS(float, rs),
+                                            WS(float, raw), out, st);
         if ((rc = launch_dec_gateup_ident(g, u, x, nullptr, M, WS(float, inter), WS(float, isum), st, D->act)))
             return rc;
         // the 8-row, 16-wave down blocks when the SwiGLU rows fit in LDS, else the per-expert one

@@ -184,6 +184,11 @@ int launch_thin_linear(const Mats& w, const uint16_t* x, int M, const float* bia
 bool thin_takes_decode(int qtype, int M, int N, int K);
 int launch_thin_decode(const Mats& w, const uint16_t* x, int M, const float* bias, void* out, int out_f16,
                        hipStream_t st);
+// A decode FFN on thin tiles (a16: 2 M rows of I halves; rs: M; raw: thin_dec_raw_bytes).
+bool thin_takes_dense_decode(const Mats& g, const Mats& u, const Mats& d, int M);
+size_t thin_dec_raw_bytes(int I, int H);
+int launch_thin_dense_decode(const Mats& g, const Mats& u, const Mats& d, const uint16_t* x, int M, int act,
+                             float* inter, uint16_t* a16, float* rs, float* raw, float* out, hipStream_t st);
 int64_t layout_bytes(int qtype, int64_t rows, int64_t cols);
 // Scale plane (relayout.hip): bytes of one matrix's plane (0 for Q8_0, -1 if unsupported)
 // and its load-time construction from the device layout.

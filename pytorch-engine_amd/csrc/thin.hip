@@ -1,4 +1,4 @@
-// Grouped products of few rows an expert (9 .. a few hundred tokens): the weights are
+// Products of few rows an expert (9 .. a few hundred tokens; some decode calls of 3 .. 8): the weights are
 // streamed once, straight from HBM into registers, and every token of a tile shares them.
 //
 // A tile is up to 32 sorted pairs of one expert (64 rows of a linear).  A block of 8 waves
@@ -44,6 +44,7 @@ typedef _Float16 th8 __attribute__((ext_vector_type(8)));
 typedef _Float16 th2 __attribute__((ext_vector_type(2)));
 typedef __bf16 tb8 __attribute__((ext_vector_type(8)));
 typedef float tf4 __attribute__((ext_vector_type(4)));
+typedef _Float16 th4 __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------- weight decode
 // Each lane turns its quarter's codes into fp16 MFMA operands with packed fp16 arithmetic
@@ -812,8 +813,9 @@ int launch_thin_down(const Mats& d, const uint16_t* a16, const float* rs, int M,
 // Q6_K 3 rows 70 -> 62, 8 rows 121 -> 64; Q4_K 56 -> 45, 103 -> 46; Q5_K 62 -> 53, 107 -> 55 (two
 // rows: Q6_K 60 -> 62).  Q8_0's d q is no fp16 value, so it stays there.  K is not split, so
 // that outputs depend on no other rows of a pack: from a block a CU on.
+static bool thin_exact(int qtype) { return qtype == PGMOE_Q4_K || qtype == PGMOE_Q5_K || qtype == PGMOE_Q6_K; }
 bool thin_takes_decode(int qtype, int M, int N, int K) {
-    return (qtype == PGMOE_Q4_K || qtype == PGMOE_Q5_K || qtype == PGMOE_Q6_K) && M > 2 && N >= 32768 && N % 4 == 0 &&
+    return thin_exact(qtype) && M > 2 && N >= 32768 && N % 4 == 0 &&
            (int64_t)M * K < ((int64_t)1 << 31);
 }
 
@@ -830,6 +832,119 @@ int launch_thin_decode(const Mats& w, const uint16_t* x, int M, const float* bia
     default: return fail(PGMOE_E_UNSUPPORTED, "thin decode linear: qtype %d", w.qtype);
     }
     return check_launch("thin linear");
+}
+
+// ---------------------------------------------------------------- decode FFN (M <= 8)
+// A dense SwiGLU FFN of 3 .. 8 tokens with K-quant matrices on thin tiles at the GEMVs' precision:
+// gate / up as the decode linear (exact weights, fp16 tokens), and the down product on the fp32
+// SwiGLU rows as two fp16 rows each, hi + mid 2^-11 with hi the rounded value and mid the rounded
+// rest (23 bits and more: the row is first brought to 2^13 .. 2^14 by a power of two), which
+// fill one 16-row tile.  Error against float64, H = 4096, I = 12288: 3.2e-5 -> 4e-7 (Q4_K, Q6_K).
+// The GEMVs' time goes with the tokens, this one's (five launches, split sums) hardly: H = 4096, I =
+// 12288, us GEMV -> here 3 tokens 63 -> 39, 4 71 -> 40, 6 98 -> 40, 8 123 -> 41; 2048 x 5632 3 tokens 17
+// -> 27, 5 22 -> 27, 8 33.5 -> 28; 1024 x 2816 8 tokens 18 -> 19: from 250 M weights times tokens on.
+constexpr int kThinDecRows = 8;
+
+bool thin_takes_dense_decode(const Mats& g, const Mats& u, const Mats& d, int M) {
+    return M > 2 && M <= kThinDecRows && thin_exact(g.qtype) && u.qtype == g.qtype && thin_exact(d.qtype) &&
+           (int64_t)M * 3 * g.N * g.K >= 250000000;
+}
+
+// Splits of K: two blocks a CU.
+static GemmSplit thin_dec_split(int N, int K) {
+    const int nb = K >> 8, s = std::min(nb, std::max(1, 512 / div_up(N, 16 * kThinWaves)));
+    const int kper = div_up(nb, s);
+    return GemmSplit{div_up(nb, kper), kper};
+}
+size_t thin_dec_raw_bytes(int I, int H) {
+    return 4 * std::max((size_t)thin_dec_split(I, H).ksplit * kThinDecRows * 2 * I,
+                        (size_t)thin_dec_split(H, I).ksplit * 2 * kThinDecRows * H);
+}
+
+// Row m of inter (I a multiple of 256) as fp16 rows m and M + m of a16; rs[m] takes them back.
+// One block a row, read twice (the second time from cache).
+__global__ __launch_bounds__(1024) void thin_rows_kernel(const float* __restrict__ inter, int M, int I,
+                                                         uint16_t* __restrict__ a16, float* __restrict__ rs) {
+    __shared__ float wmx[16];
+    const int tid = threadIdx.x, m = blockIdx.x, n4 = I >> 2;
+    const float4* row = (const float4*)(inter + (int64_t)m * I);
+    float mx = 0.f;
+    for (int i = tid; i < n4; i += 1024) {
+        const float4 v = row[i];
+        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+    }
+    mx = wave_max(mx);
+    if ((tid & 63) == 0) wmx[tid >> 6] = mx;
+    __syncthreads();
+    mx = wmx[0];
+    for (int w = 1; w < 16; ++w) mx = fmaxf(mx, wmx[w]);
+    // 2^k, k = 13 - exponent(mx), within +-110 (a zero row, an infinite one: any finite scale)
+    const int k = max(-110, min(110, 140 - (int)((__builtin_bit_cast(uint32_t, mx) >> 23) & 0xff)));
+    const float sc = __builtin_bit_cast(float, (uint32_t)(127 + k) << 23);
+    if (tid == 0) rs[m] = __builtin_bit_cast(float, (uint32_t)(127 - k) << 23);
+    th4* hi = (th4*)(a16 + (int64_t)m * I);
+    th4* mid = (th4*)(a16 + (int64_t)(M + m) * I);
+    for (int i = tid; i < n4; i += 1024) {
+        const float4 v = row[i];
+        const float a[4] = {v.x * sc, v.y * sc, v.z * sc, v.w * sc};
+        th4 h, r;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            h[c] = (_Float16)a[c];
+            r[c] = (_Float16)((a[c] - (float)h[c]) * 2048.0f);
+        }
+        hi[i] = h;
+        mid[i] = r;
+    }
+}
+
+// out[m] = rs[m] (sum of row m's splits + 2^-11 of row M + m's), in split order.
+__global__ __launch_bounds__(256) void thin_rows_reduce_kernel(const float* __restrict__ raw, int S, int M, int N,
+                                                               const float* __restrict__ rs, float* __restrict__ out) {
+    const int i = blockIdx.x * 256 + threadIdx.x, N4 = N >> 2;
+    if (i >= M * N4) return;
+    const int m = i / N4, c = i - m * N4;
+    const tf4* r = (const tf4*)raw + (int64_t)m * N4 + c;
+    tf4 a{0.f, 0.f, 0.f, 0.f}, b = a;
+#pragma unroll 4
+    for (int s = 0; s < S; ++s) {
+        a = a + r[(int64_t)s * 2 * M * N4];
+        b = b + r[((int64_t)s * 2 + 1) * M * N4];
+    }
+    ((tf4*)out)[i] = rs[m] * (a + b * (1.0f / 2048.0f));
+}
+
+template <bool GATEUP>
+static int thin_dec_launch(int qtype, ThinArgs& a, hipStream_t st) {
+    const GemmSplit sp = thin_dec_split(a.N, a.K);
+    a.kper = sp.kper;
+    const dim3 grid(div_up(a.N, 16 * kThinWaves), 1, sp.ksplit);
+    constexpr int R = GATEUP ? 2 : 1;
+    switch (qtype) {
+    case PGMOE_Q4_K: PG_LAUNCH((thin_kernel<PGMOE_Q4_K, GATEUP, R, 1>), grid, dim3(kThinThreads), 0, st, a); break;
+    case PGMOE_Q5_K: PG_LAUNCH((thin_kernel<PGMOE_Q5_K, GATEUP, R, 1>), grid, dim3(kThinThreads), 0, st, a); break;
+    case PGMOE_Q6_K: PG_LAUNCH((thin_kernel<PGMOE_Q6_K, GATEUP, R, 1>), grid, dim3(kThinThreads), 0, st, a); break;
+    default: return fail(PGMOE_E_UNSUPPORTED, "thin decode: qtype %d", qtype);
+    }
+    return check_launch("thin decode");
+}
+
+int launch_thin_dense_decode(const Mats& g, const Mats& u, const Mats& d, const uint16_t* x, int M, int act,
+                             float* inter, uint16_t* a16, float* rs, float* raw, float* out, hipStream_t st) {
+    ThinArgs a{};
+    a.w0 = g.base, a.w1 = u.base, a.N = g.N, a.K = g.K, a.act = x, a.topk = 1, a.P = M;
+    a.out = inter, a.act_kind = act, a.raw = raw;
+    int rc = thin_dec_launch<true>(g.qtype, a, st);
+    if (rc) return rc;
+    const int S = thin_dec_split(g.N, g.K).ksplit;
+    if ((rc = launch_split_reduce(1, raw, S, M, g.N, nullptr, nullptr, nullptr, inter, st, act))) return rc;
+    PG_LAUNCH(thin_rows_kernel, dim3(M), dim3(1024), 0, st, inter, M, g.N, a16, rs);
+    ThinArgs b{};
+    b.w0 = d.base, b.N = d.N, b.K = d.K, b.act = a16, b.topk = 1, b.P = 2 * M, b.raw = raw;
+    if ((rc = thin_dec_launch<false>(d.qtype, b, st))) return rc;
+    PG_LAUNCH(thin_rows_reduce_kernel, dim3(div_up(M * (d.N >> 2), 256)), dim3(256), 0, st, raw,
+              thin_dec_split(d.N, d.K).ksplit, M, d.N, rs, out);
+    return check_launch("thin decode reduce");
 }
 
 int launch_thin_linear(const Mats& w, const uint16_t* x, int M, const float* bias, void* out, int out_f16, float* raw,

@@ -98,6 +98,30 @@ def test_layer_tiles(gate_up, down):
         check_layer_output(got, ol.forward_tokens(x, idx, w))
 
 
+@pytest.mark.parametrize("gate_up,down", [(Q4_K, Q6_K), (Q5_K, Q4_K), (Q6_K, Q5_K)])
+@pytest.mark.parametrize("H,I", [(256, 108800), (2304, 12544), (12544, 2304)])
+def test_decode_dense_on_thin_tiles(gate_up, down, H, I):
+    """3 .. 8 tokens against float64 on the decoded weights: gate and up within 5.4e-6 of their
+    norms as above, their product and the down sums the same again, the split rows 2^-22: 2e-5 of
+    the result's norm in all.  Rows that differ by 2^16 in size keep their own accuracy."""
+    from pgmoe import HipDenseMLP
+    dev = torch.device("cuda", 0)
+    lay = SyntheticDense(DenseSpec("thin", H, I, (gate_up, gate_up, down)), seed=3, scale=0.01)
+    mod = HipDenseMLP(lay.gguf, lay.config, 0, dev)
+    g, u, d = (torch.from_numpy(oracle.dequant(t.qtype, lay.tensor(f"ffn_{p}.weight"), *t.shape)).to(dev).double()
+               for p in ("gate", "up", "down") for t in [lay.gguf.tensors[f"blk.0.ffn_{p}.weight"]])
+    x = torch.from_numpy(lay.draw_x(9)).to(dev)
+    x[1] *= 2.0 ** -8
+    x[2] = 0
+    ref = (torch.nn.functional.silu(x.double() @ g.T) * (x.double() @ u.T)) @ d.T
+    for M in (3, 5, 8):
+        log(f"thin decode dense {gate_up}/{down} H={H} I={I} M={M}")
+        got = mod(x[:M].clone()).double()
+        assert torch.all(got[2] == 0)
+        err = (got - ref[:M]).norm(dim=1) / ref[:M].norm(dim=1).clamp_min(1e-300)
+        assert float(err.max()) <= 2e-5, (M, err)
+
+
 def test_dense_sides_of_the_rule_and_replays():
     """Both products on thin tiles, only the down one, and neither; a captured forward on thin
     tiles equals the eager one at every replay."""
