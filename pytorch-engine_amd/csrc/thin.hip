@@ -397,7 +397,8 @@ struct ThinArgs {
     float* raw;                  // split K: raw sums [split][P][NC]
 };
 
-// A finite fp32 value as three bf16 pieces that add up to it, then a zero.
+// A finite fp32 value as three bf16 pieces that add up to it, then a zero.  An infinity or NaN
+// gives NaN, which thin_non_finite takes back where the call has to.
 __device__ __forceinline__ u32x2 thin_split3(float v) {
     const uint32_t a = __builtin_bit_cast(uint32_t, v) & 0xffff0000u;
     const float r = v - __builtin_bit_cast(float, a);
@@ -489,13 +490,53 @@ __device__ __forceinline__ void thin_block(const ThinConst& kc, const uint8_t* x
     }
 }
 
+// Element k (from super-block tile t on) of a Q4_K / Q5_K row as the 256-row tiles hold it, rounded
+// to fp16 (off0: the row's 16 bytes).
+template <int QT>
+__device__ __forceinline__ float thin_weight(const uint8_t* t, uint32_t off0, int k) {
+    t += (int64_t)(k >> 8) * (Tile<QT>::CH * 1024) + off0;
+    const int s = (k >> 5) & 7, l = k & 31, j = 32 * (s >> 1) + l;  // sub-block, element of it, byte of qs
+    const u32x4 h = ldq(t);
+    int sc, mn, q = (t[(1 + (j >> 4)) * 1024 + (j & 15)] >> (4 * (s & 1))) & 15;
+    if constexpr (QT == PGMOE_Q5_K) q |= ((t[(9 + (s >> 2)) * 1024 + 4 * (s & 3) + (l & 3)] >> (l >> 2)) & 1) << 4;
+    kscale_sel(h.y, h.z, h.w, s, sc, mn);
+    const float a = lo_half(h.x) * (float)sc, c = -(hi_half(h.x) * (float)mn) - 1024.0f * a;
+    return (float)(_Float16)__builtin_fmaf(1024.0f + (float)q, a, c);
+}
+
+// The sums of a Q4_K / Q5_K token with an infinity or NaN are NaN here (the codes and the minima
+// are products of their own: inf - inf, or inf times a zero code), where the sum of x w is +-inf
+// wherever the terms that are not finite agree.  So where the K elements at x hold such terms, f
+// is their sum alone, with the weights (weight(r, k): row tile r's, element k) rounded to fp16 as
+// the 256-row tiles round them.  Runs only in waves that hold a NaN.
+template <int R, class Weight>
+__device__ __forceinline__ bool thin_non_finite(const uint16_t* x, int K, const Weight& weight, float (&f)[R]) {
+    bool hit = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r) f[r] = 0.f;
+#pragma unroll 1
+    for (int k = 0; k < K; k += 8) {
+        const u32x4 v = ldq((const uint8_t*)(x + k));
+#pragma unroll 1
+        for (int c = 0; c < 8; ++c) {
+            const uint32_t w = c < 4 ? (c < 2 ? v.x : v.y) : (c < 6 ? v.z : v.w);
+            const uint16_t b = (uint16_t)(w >> (16 * (c & 1)));
+            if ((b & 0x7c00) != 0x7c00) continue;
+            hit = true;
+#pragma unroll
+            for (int r = 0; r < R; ++r) f[r] = __builtin_fmaf(h2f(b), weight(r, k + c), f[r]);
+        }
+    }
+    return hit;
+}
+
 // A wave's part of a tile of n <= 16 NT pairs from m0: the K loop and the epilogue (a whole
 // copy a token-tile count, so that one's registers never meet another's).  smem: two stages
-// of rows, then two of sums.
-template <int QT, bool GATEUP, int R, int NT, bool EX, class Load>
+// of rows, then two of sums.  weight: thin_non_finite's.
+template <int QT, bool GATEUP, int R, int NT, bool EX, class Load, class Weight>
 __device__ __forceinline__ void thin_tile(const ThinArgs& A, uint8_t* smem, const uint32_t* rowsrc, const float* rowscale,
                                           const ThinConst& kc, int m0, int n, int row0, int b0, int nsb,
-                                          Qtr<QT> (&q)[R], Load& load) {
+                                          Qtr<QT> (&q)[R], Load& load, const Weight& weight) {
     using S = ThinStage<NT>;
     using W = ThinW<QT>;
     constexpr int CP = 16 * NT * S::PIECES / kThinThreads / S::SPB;  // 16-byte copies a thread and super-block step
@@ -581,35 +622,54 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& A, uint8_t* smem, cons
 
     // lane l: output column row0 (+ 16 r) + l % 16 of tokens 16 t + 4 (l / 16) + 0..3
     const int col = row0 + (lane & 15);
+    auto emit = [&](int tok, const float (&sum)[R]) {
+        const int64_t pr = m0 + tok;
+        if (A.raw) {
+            const int NC = GATEUP ? 2 * A.N : A.N;
+            float* rb = A.raw + ((int64_t)blockIdx.z * A.P + pr) * NC + col;
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (col + (GATEUP ? 0 : 16 * r) < A.N) rb[GATEUP ? r * A.N : 16 * r] = sum[r];
+        } else if constexpr (GATEUP) {
+            if (col < A.N) ((float*)A.out)[pr * A.N + col] = thin_act(A.act_kind, sum[0]) * sum[1];
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int c = col + 16 * r;
+                if (c >= A.N) continue;
+                float o = sum[r] * rowscale[tok];
+                if (A.bias) o += A.bias[c];
+                if (A.out_f16)
+                    ((_Float16*)A.out)[pr * A.N + c] = (_Float16)o;
+                else
+                    ((float*)A.out)[pr * A.N + c] = o;
+            }
+        }
+    };
+    bool nan = false;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int tok = 16 * t + 4 * p + v;
-            if (tok >= n) continue;
-            const int64_t pr = m0 + tok;
-            if (A.raw) {
-                const int NC = GATEUP ? 2 * A.N : A.N;
-                float* rb = A.raw + ((int64_t)blockIdx.z * A.P + pr) * NC + col;
+            float sum[R];
 #pragma unroll
-                for (int r = 0; r < R; ++r)
-                    if (col + (GATEUP ? 0 : 16 * r) < A.N) rb[GATEUP ? r * A.N : 16 * r] = acc[r][t][v];
-            } else if constexpr (GATEUP) {
-                if (col < A.N) ((float*)A.out)[pr * A.N + col] = thin_act(A.act_kind, acc[0][t][v]) * acc[1][t][v];
-            } else {
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const int c = col + 16 * r;
-                    if (c >= A.N) continue;
-                    float o = acc[r][t][v] * rowscale[tok];
-                    if (A.bias) o += A.bias[c];
-                    if (A.out_f16)
-                        ((_Float16*)A.out)[pr * A.N + c] = (_Float16)o;
-                    else
-                        ((float*)A.out)[pr * A.N + c] = o;
-                }
+            for (int r = 0; r < R; ++r) {
+                sum[r] = acc[r][t][v];
+                nan |= sum[r] != sum[r];
             }
+            if (tok < n) emit(tok, sum);
         }
+    // (not in the decode GEMVs' place, EX: they give NaN for such tokens too)
+    if constexpr (W::MINS && !EX) {
+        if (!__any(nan)) return;
+#pragma unroll 1
+        for (int i = 0; i < 4 * NT; ++i) {
+            const int tok = 16 * (i >> 2) + 4 * p + (i & 3);
+            float sum[R];
+            if (tok < n && thin_non_finite(A.act + rowsrc[tok] + 256 * b0, 256 * nsb, weight, sum)) emit(tok, sum);
+        }
+    }
 }
 
 // Tiles of up to 16 MAXNT pairs; R row tiles a wave (gate/up: gate and up rows).  MAXNT 1: a
@@ -656,21 +716,30 @@ __global__ __launch_bounds__(kThinThreads, 4) void thin_kernel(const ThinArgs A)
     const int row0 = ((int)blockIdx.x * kThinWaves + wave) * (GATEUP ? 16 : 16 * R);
     const int p = lane >> 4;
     const int ngr = row_groups(A.N);
+    auto row_tile = [&](int first, int r, const uint8_t*& t, const uint8_t*& d) {
+        const uint8_t* mat = GATEUP && r ? A.w1 + (int64_t)e * A.stride1 : A.w0 + (int64_t)e * A.stride0;
+        const int row = min(GATEUP ? first : first + 16 * r, 64 * ngr - 16);
+        const int64_t g = (int64_t)(row >> 6) * nb + b0;
+        t = mat + g * (Tile<QT>::CH * 1024) + (row & 63) * 16;
+        d = mat + (int64_t)ngr * nb * (Tile<QT>::CH * 1024) + (g * 64 + (row & 63)) * 2;
+    };
     const uint8_t *tb[R], *db[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const uint8_t* mat = GATEUP && r ? A.w1 + (int64_t)e * A.stride1 : A.w0 + (int64_t)e * A.stride0;
-        const int row = min(GATEUP ? row0 : row0 + 16 * r, 64 * ngr - 16);
-        const int64_t g = (int64_t)(row >> 6) * nb + b0;
-        tb[r] = mat + g * (Tile<QT>::CH * 1024) + (row & 63) * 16;
-        db[r] = mat + (int64_t)ngr * nb * (Tile<QT>::CH * 1024) + (g * 64 + (row & 63)) * 2;
-    }
+    for (int r = 0; r < R; ++r) row_tile(row0, r, tb[r], db[r]);
     Qtr<QT> q[R];
     const ThinConst kc = thin_const<QT>(p);
     uint32_t off0, offp;
     thin_offsets<QT>(lane, p, off0, offp);
     auto load = [&](int r, int b) {  // super-block b < nsb of the split
         thin_load<QT>(q[r], tb[r] + (uint32_t)b * (Tile<QT>::CH * 1024), db[r] + b * 128, off0, offp, lane, p);
+    };
+    auto weight = [&](int r, int k) {  // (its tile found anew: kept through the K loop it costs registers)
+        int first = row0;
+        asm volatile("" : "+s"(first));
+        const uint8_t *t, *d;
+        row_tile(first, r, t, d);
+        if constexpr (ThinW<QT>::MINS) return thin_weight<QT>(t, 16 * (threadIdx.x & 15), k);
+        else return 0.f;
     };
 #pragma unroll
     for (int r = 0; r < R; ++r) load(r, 0);
@@ -682,10 +751,10 @@ __global__ __launch_bounds__(kThinThreads, 4) void thin_kernel(const ThinArgs A)
     __syncthreads();
 
     const int nt = (n + 15) >> 4;
-    if (MAXNT == 1 || nt == 1) thin_tile<QT, GATEUP, R, 1, MAXNT == 1>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load);
+    if (MAXNT == 1 || nt == 1) thin_tile<QT, GATEUP, R, 1, MAXNT == 1>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load, weight);
     else if constexpr (MAXNT > 1) {
-        if (nt == 2) thin_tile<QT, GATEUP, R, 2, false>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load);
-        else if constexpr (MAXNT > 2) thin_tile<QT, GATEUP, R, 4, false>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load);
+        if (nt == 2) thin_tile<QT, GATEUP, R, 2, false>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load, weight);
+        else if constexpr (MAXNT > 2) thin_tile<QT, GATEUP, R, 4, false>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load, weight);
     }
 }
 

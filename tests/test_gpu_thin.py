@@ -151,3 +151,38 @@ def test_dense_sides_of_the_rule_and_replays():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, mod(x))
+
+
+@pytest.mark.parametrize("qt", [Q4_1, Q8_0, Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("N,K", [(68, 256), (260, 1280), (4100, 512)])
+def test_tokens_that_are_not_finite(qt, N, K):
+    """Infinities in a token give what the sum over their terms gives with the weights rounded to
+    fp16 (+-inf where they agree in sign, else NaN), a NaN gives NaN, and the other tokens of the
+    tile are bit-equal to a run without them.  Weights near zero, whose sign the rounding of the
+    decoded value decides, are left out."""
+    from pgmoe import GGUFQuantLinear
+    dev = torch.device("cuda", 0)
+    rng = np.random.default_rng(N + K + qt)
+    raw = random_blocks(rng, qt, N, K, 0.01)
+    lin = GGUFQuantLinear("w8", K, N, qt, raw=raw, device=dev)
+    w = oracle.dequant(qt, raw, N, K)
+    x = rng.standard_normal((65, K)).astype(np.float16)
+    bad = x.copy()
+    terms = {3: {7: np.inf}, 8: {K - 1: -np.inf}, 16: {40: np.inf, 200: np.inf}, 32: {0: np.inf, 131: -np.inf}}
+    for t, at in terms.items():
+        for k, v in at.items():
+            bad[t, k] = v
+    bad[5, 99] = np.nan
+    touched = np.isin(np.arange(65), [*terms, 5])
+    for M in (9, 17, 33, 65):
+        log(f"thin non-finite qt={qt} N={N} K={K} M={M}")
+        clean = lin(torch.from_numpy(x[:M]).to(dev).float()).cpu().numpy()
+        got = lin(torch.from_numpy(bad[:M]).to(dev).float()).cpu().numpy()
+        assert np.array_equal(got[~touched[:M]], clean[~touched[:M]])
+        assert np.all(np.isnan(got[5]))
+        for t, at in terms.items():
+            if t < M:
+                cols = np.all([np.abs(w[:, k]) > 1e-3 * np.abs(w).max() for k in at], axis=0)
+                with np.errstate(invalid="ignore"):
+                    ref = sum(w[:, k].astype(np.float16) * np.float16(v) for k, v in at.items())
+                assert cols.sum() > N // 4 and np.array_equal(got[t, cols], ref[cols], equal_nan=True), (M, t)
