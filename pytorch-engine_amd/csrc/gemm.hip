@@ -715,14 +715,15 @@ __global__ __launch_bounds__(64 * (WM * 8 / CT)) void gemm_kernel(
 // the same order run at streaming rate.  Measured (Qwen2 shared expert's down product,
 // M = 512): one column a thread 17.3 us, four 13.2 us.
 constexpr int kMaxSplitLoads = 8;
-// KIND 0: down, 1: gate/up, 2: linear (rs = the bias or null, act = fp16 output).
+// KIND 0: down, 1: gate/up, 2: linear (rs = the bias or null, act = fp16 output), 3: gate/up with
+// the decode kernels' activation (expf and a division).
 template <int KIND>
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const float* __restrict__ raw, int S, int64_t P,
                                                                 int N, const float* __restrict__ rs,
                                                                 const float* __restrict__ topk_w,
                                                                 const int32_t* __restrict__ perm,
                                                                 void* __restrict__ outv, int act) {
-    constexpr bool GATEUP = KIND == 1;
+    constexpr bool GATEUP = KIND == 1 || KIND == 3;
     float* out = (float*)outv;
     const int N4 = N >> 2;
     const int64_t n4 = P * N4;
@@ -761,7 +762,10 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const float* __r
                 }
         }
         float4 o;
-        if constexpr (GATEUP) {
+        if constexpr (KIND == 3) {
+            o = make_float4(gate_act(act, a.x) * b.x, gate_act(act, a.y) * b.y, gate_act(act, a.z) * b.z,
+                            gate_act(act, a.w) * b.w);
+        } else if constexpr (GATEUP) {
             o = make_float4(act_fast(act, a.x) * b.x, act_fast(act, a.y) * b.y, act_fast(act, a.z) * b.z,
                             act_fast(act, a.w) * b.w);
         } else if constexpr (KIND == 0) {
@@ -857,6 +861,7 @@ int launch_split_reduce(int kind, const float* raw, int S, int64_t P, int N, con
     PG_LAUNCH(gemm_split_reduce_kernel<KIND>, dim3(blocks), dim3(256), 0, st, raw, S, P, N, rs, topk_w, perm, out, act)
     if (kind == 1) PG_SR(1);
     else if (kind == 0) PG_SR(0);
+    else if (kind == 3) PG_SR(3);
     else PG_SR(2);
 #undef PG_SR
     return check_launch("gemm split reduce");

@@ -164,7 +164,8 @@ size_t gemm_split_bytes(int64_t P, int E, int N, int K, bool gateup);
 size_t gemm_split_bytes_upto(int64_t P, int E, int N, int K, bool gateup);
 int gemm_tile_pairs();
 // The S raw partial sums [split][P][N] (gate/up: 2N) added in split order, then the epilogue
-// of kind 0 (down), 1 (gate/up, act) or 2 (linear: rs = bias or null, act = fp16 output).
+// of kind 0 (down), 1 (gate/up, act), 2 (linear: rs = bias or null, act = fp16 output) or 3
+// (gate/up, act as the decode kernels compute it).
 int launch_split_reduce(int kind, const float* raw, int S, int64_t P, int N, const float* rs, const float* topk_w,
                         const int32_t* perm, void* out, hipStream_t st, int act);
 // Products of few rows an expert (thin.hip), on tiles of thin_tile_rows() pairs; the same

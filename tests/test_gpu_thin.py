@@ -186,3 +186,52 @@ def test_tokens_that_are_not_finite(qt, N, K):
                 with np.errstate(invalid="ignore"):
                     ref = sum(w[:, k].astype(np.float16) * np.float16(v) for k, v in at.items())
                 assert cols.sum() > N // 4 and np.array_equal(got[t, cols], ref[cols], equal_nan=True), (M, t)
+
+
+def _int_ffn(gate, up, down, arch="qwen3"):
+    """A dense FFN of whole-number weights: gate and up [I, H] (0 .. 15) as Q4_K, down [H, I] (-32 ..
+    31) as Q6_K, every scale 1 and every minimum 0."""
+    from pgmoe import HipDenseMLP
+    from pgmoe.gguf import InMemoryGGUF
+
+    def q4(c):
+        c = c.reshape(-1, 4, 2, 32).astype(np.uint8)
+        qs = (c[:, :, 0] | (c[:, :, 1] << 4)).reshape(-1, 128)
+        head = np.frombuffer(np.float16(1).tobytes() + bytes(2) + bytes([1] * 4 + [0] * 4 + [1] * 4), np.uint8)
+        return np.concatenate([np.broadcast_to(head, (len(qs), 16)), qs], 1)
+
+    def q6(c):
+        c = (c + 32).reshape(-1, 2, 4, 32).astype(np.uint8)
+        ql = np.concatenate([(c[:, :, 0] & 15) | ((c[:, :, 2] & 15) << 4), (c[:, :, 1] & 15) | ((c[:, :, 3] & 15) << 4)], 2)
+        qh = sum((c[:, :, s] >> 4) << (2 * s) for s in range(4))
+        tail = np.frombuffer(bytes([1] * 16) + np.float16(1).tobytes(), np.uint8)
+        return np.concatenate([ql.reshape(-1, 128), qh.reshape(-1, 64), np.broadcast_to(tail, (len(ql), 18))], 1)
+
+    I, H = gate.shape
+    g = InMemoryGGUF({"general.architecture": arch, f"{arch}.embedding_length": H, f"{arch}.feed_forward_length": I})
+    g.add_tensor("blk.0.ffn_gate.weight", (I, H), Q4_K, q4(gate))
+    g.add_tensor("blk.0.ffn_up.weight", (I, H), Q4_K, q4(up))
+    g.add_tensor("blk.0.ffn_down.weight", (H, I), Q6_K, q6(down))
+    return HipDenseMLP(g, g.build_model_config(), 0, torch.device("cuda", 0))
+
+
+@pytest.mark.parametrize("arch", ["qwen3", "gemma3"])
+def test_decode_dense_activation(arch):
+    """Each output is one activation times a whole number.  SiLU of -38 .. -3 in fp32: expf 2^-23,
+    1 + x, the quotient and the product 2^-24 each, the rows' pieces and their sum 2^-23: 4.2e-7
+    (the hardware exp2 of a rounded argument is off by up to 2.4e-6 alone).  GELU of 3 .. 38:
+    2z to 4 x 2^-24 of itself, which moves 1 - 1 / (1 + e^2z) by at most 0.3 of that; 1e-6."""
+    H, I, M = 1024, 10240, 8
+    gate, up, down = np.zeros((I, H), np.int64), np.zeros((I, H), np.int64), np.zeros((H, I), np.int64)
+    i, h = np.arange(I), np.arange(H)
+    gate[:, 0], up[:, 1] = 12 + i % 4, 1 + i % 7  # (a row's values within 2^12 of one another)
+    at = (10 * h + 3 * (h // 64)) % I
+    down[h, at] = 1
+    x = np.zeros((M, H), np.float16)
+    x[:, 0] = (1 if arch == "gemma3" else -1) * np.array([0.25, 0.5, 0.75, 1, 1.25, 1.75, 2, 2.5])
+    x[:, 1] = 1
+    got = _int_ffn(gate, up, down, arch)(torch.from_numpy(x).to("cuda:0")).double().cpu()
+    g = torch.from_numpy(x[:, :1].astype(np.float64) * gate[at, 0])
+    a = torch.nn.functional.gelu(g, approximate="tanh") if arch == "gemma3" else torch.nn.functional.silu(g)
+    ref = a * torch.from_numpy(up[at, 1].astype(np.float64))
+    assert float(((got - ref) / ref).abs().max()) <= (1e-6 if arch == "gemma3" else 6e-7)
