@@ -210,7 +210,7 @@ static DenseLayout dense_layout(int M, int I, int H) {
     o.w = take(c, gemm ? (size_t)M * 4 : 0);
     o.inter = take(c, (size_t)M * I * 4);
     o.isum = take(c, gemm ? 0 : (size_t)M * (I / 16) * 4);
-    o.a16 = take(c, (size_t)(gemm ? M : 2 * M) * I * 2);  // decode: two rows a token
+    o.a16 = take(c, (size_t)(gemm ? M : 3 * M) * I * 2);  // decode: three rows a token
     o.rs = take(c, (size_t)M * 4);
     o.raw = take(c, gemm ? std::max(gemm_split_bytes_upto(M, 1, I, H, true), gemm_split_bytes_upto(M, 1, H, I, false))
                          : M > 2 ? thin_dec_raw_bytes(I, H) : 0);

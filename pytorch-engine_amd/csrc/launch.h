@@ -185,7 +185,7 @@ int launch_thin_linear(const Mats& w, const uint16_t* x, int M, const float* bia
 bool thin_takes_decode(int qtype, int M, int N, int K);
 int launch_thin_decode(const Mats& w, const uint16_t* x, int M, const float* bias, void* out, int out_f16,
                        hipStream_t st);
-// A decode FFN on thin tiles (a16: 2 M rows of I halves; rs: M; raw: thin_dec_raw_bytes).
+// A decode FFN on thin tiles (a16: 3 M rows of I halves; rs: M; raw: thin_dec_raw_bytes).
 bool thin_takes_dense_decode(const Mats& g, const Mats& u, const Mats& d, int M);
 size_t thin_dec_raw_bytes(int I, int H);
 int launch_thin_dense_decode(const Mats& g, const Mats& u, const Mats& d, const uint16_t* x, int M, int act,

@@ -672,9 +672,9 @@ __device__ __forceinline__ void thin_tile(const ThinArgs& A, uint8_t* smem, cons
     }
 }
 
-// Tiles of up to 16 MAXNT pairs; R row tiles a wave (gate/up: gate and up rows).  MAXNT 1: a
-// decode linear (EX: exact weights).
-template <int QT, bool GATEUP, int R, int MAXNT>
+// Tiles of up to 16 MAXNT pairs; R row tiles a wave (gate/up: gate and up rows).  EX: exact weights,
+// for the decode calls.
+template <int QT, bool GATEUP, int R, int MAXNT, bool EX = false>
 __global__ __launch_bounds__(kThinThreads, 4) void thin_kernel(const ThinArgs A) {
     constexpr int ROWS = 16 * MAXNT;
     static_assert(!GATEUP || R == 2, "gate/up: a gate and an up row tile a wave");
@@ -751,10 +751,10 @@ __global__ __launch_bounds__(kThinThreads, 4) void thin_kernel(const ThinArgs A)
     __syncthreads();
 
     const int nt = (n + 15) >> 4;
-    if (MAXNT == 1 || nt == 1) thin_tile<QT, GATEUP, R, 1, MAXNT == 1>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load, weight);
+    if (MAXNT == 1 || nt == 1) thin_tile<QT, GATEUP, R, 1, EX>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load, weight);
     else if constexpr (MAXNT > 1) {
-        if (nt == 2) thin_tile<QT, GATEUP, R, 2, false>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load, weight);
-        else if constexpr (MAXNT > 2) thin_tile<QT, GATEUP, R, 4, false>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load, weight);
+        if (nt == 2) thin_tile<QT, GATEUP, R, 2, EX>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load, weight);
+        else if constexpr (MAXNT > 2) thin_tile<QT, GATEUP, R, 4, EX>(A, smem, rowsrc, rowscale, kc, m0, n, row0, b0, nsb, q, load, weight);
     }
 }
 
@@ -895,24 +895,27 @@ int launch_thin_decode(const Mats& w, const uint16_t* x, int M, const float* bia
     a.bias = bias, a.out = out, a.out_f16 = out_f16, a.kper = w.K >> 8;
     const dim3 grid(div_up(a.N, 16 * kThinWaves), 1, 1);
     switch (w.qtype) {
-    case PGMOE_Q4_K: PG_LAUNCH((thin_kernel<PGMOE_Q4_K, false, 1, 1>), grid, dim3(kThinThreads), 0, st, a); break;
-    case PGMOE_Q5_K: PG_LAUNCH((thin_kernel<PGMOE_Q5_K, false, 1, 1>), grid, dim3(kThinThreads), 0, st, a); break;
-    case PGMOE_Q6_K: PG_LAUNCH((thin_kernel<PGMOE_Q6_K, false, 1, 1>), grid, dim3(kThinThreads), 0, st, a); break;
+    case PGMOE_Q4_K: PG_LAUNCH((thin_kernel<PGMOE_Q4_K, false, 1, 1, true>), grid, dim3(kThinThreads), 0, st, a); break;
+    case PGMOE_Q5_K: PG_LAUNCH((thin_kernel<PGMOE_Q5_K, false, 1, 1, true>), grid, dim3(kThinThreads), 0, st, a); break;
+    case PGMOE_Q6_K: PG_LAUNCH((thin_kernel<PGMOE_Q6_K, false, 1, 1, true>), grid, dim3(kThinThreads), 0, st, a); break;
     default: return fail(PGMOE_E_UNSUPPORTED, "thin decode linear: qtype %d", w.qtype);
     }
     return check_launch("thin linear");
 }
 
 // ---------------------------------------------------------------- decode FFN (M <= 8)
-// A dense SwiGLU FFN of 3 .. 8 tokens with K-quant matrices on thin tiles at the GEMVs' precision:
-// gate / up as the decode linear (exact weights, fp16 tokens), the GEMVs' activation (expf and a
-// division; the hardware forms cost 2e-6 of it at -38 and save 0.3 us), and the down product on the fp32
-// SwiGLU rows as two fp16 rows each, hi + mid 2^-11 with hi the rounded value and mid the rounded
-// rest (23 bits and more: the row is first brought to 2^13 .. 2^14 by a power of two), which
-// fill one 16-row tile.  Error against float64, H = 4096, I = 12288: 3.2e-5 -> 4e-7 (Q4_K, Q6_K).
+// A dense SwiGLU FFN of 3 .. 8 tokens with K-quant matrices on thin tiles: gate / up as the decode
+// linear (exact weights, fp16 tokens), the GEMVs' activation (expf and a division; the hardware
+// forms cost 2e-6 of it at -38 and save 0.3 us), and the down product on the fp32 SwiGLU rows as three
+// fp16 rows each, hi + mid 2^-11 + lo 2^-22, each piece the rounded rest of the ones before.  A row
+// is first brought to 2^13 .. 2^14 by a power of two, so that values within 2^-36 of its largest keep
+// their 24 bits and every value 2^-60 of the largest.  (Two pieces hold 23 bits; 4 tokens 41.4 us with
+// two, 42.0 with three, 8 tokens 42.6 and 44.9.)  Up to 5 tokens fill one 16-row tile, 6 .. 8 two.
+// Error against float64, H = 4096, I = 12288: 3.2e-5 -> 4e-7 (Q4_K, Q6_K).
 // The GEMVs' time goes with the tokens, this one's (five launches, split sums) hardly: H = 4096, I =
-// 12288, us GEMV -> here 3 tokens 63 -> 39, 4 71 -> 40, 6 98 -> 40, 8 123 -> 41; 2048 x 5632 3 tokens 17
-// -> 27, 5 22 -> 27, 8 33.5 -> 28; 1024 x 2816 8 tokens 18 -> 19: from 250 M weights times tokens on.
+// 12288, us GEMV -> here 3 tokens 63 -> 42, 4 71 -> 42, 6 98 -> 44, 8 123 -> 45; 2048 x 11264 4 tokens 52
+// -> 35; with two pieces 2048 x 5632 3 tokens 17 -> 27, 5 22 -> 27, 8 33.5 -> 28; 1024 x 2816 8 tokens
+// 18 -> 19: from 250 M weights times tokens on.
 constexpr int kThinDecRows = 8;
 
 bool thin_takes_dense_decode(const Mats& g, const Mats& u, const Mats& d, int M) {
@@ -928,10 +931,10 @@ static GemmSplit thin_dec_split(int N, int K) {
 }
 size_t thin_dec_raw_bytes(int I, int H) {
     return 4 * std::max((size_t)thin_dec_split(I, H).ksplit * kThinDecRows * 2 * I,
-                        (size_t)thin_dec_split(H, I).ksplit * 2 * kThinDecRows * H);
+                        (size_t)thin_dec_split(H, I).ksplit * 3 * kThinDecRows * H);
 }
 
-// Row m of inter (I a multiple of 256) as fp16 rows m and M + m of a16; rs[m] takes them back.
+// Row m of inter (I a multiple of 256) as fp16 rows m, M + m and 2M + m of a16; rs[m] takes them back.
 // One block a row, read twice (the second time from cache).
 __global__ __launch_bounds__(1024) void thin_rows_kernel(const float* __restrict__ inter, int M, int I,
                                                          uint16_t* __restrict__ a16, float* __restrict__ rs) {
@@ -948,52 +951,67 @@ __global__ __launch_bounds__(1024) void thin_rows_kernel(const float* __restrict
     __syncthreads();
     mx = wmx[0];
     for (int w = 1; w < 16; ++w) mx = fmaxf(mx, wmx[w]);
-    // 2^k, k = 13 - exponent(mx), within +-110 (a zero row, an infinite one: any finite scale)
-    const int k = max(-110, min(110, 140 - (int)((__builtin_bit_cast(uint32_t, mx) >> 23) & 0xff)));
+    // 2^k, k = 13 - exponent(mx), -115 .. 126 (so that 2^-k is normal; a zero row: any scale)
+    const int k = min(126, 140 - (int)((__builtin_bit_cast(uint32_t, mx) >> 23) & 0xff));
     const float sc = __builtin_bit_cast(float, (uint32_t)(127 + k) << 23);
     if (tid == 0) rs[m] = __builtin_bit_cast(float, (uint32_t)(127 - k) << 23);
     th4* hi = (th4*)(a16 + (int64_t)m * I);
     th4* mid = (th4*)(a16 + (int64_t)(M + m) * I);
+    th4* lo = (th4*)(a16 + (int64_t)(2 * M + m) * I);
     for (int i = tid; i < n4; i += 1024) {
         const float4 v = row[i];
         const float a[4] = {v.x * sc, v.y * sc, v.z * sc, v.w * sc};
-        th4 h, r;
+        th4 h, r, l;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             h[c] = (_Float16)a[c];
-            r[c] = (_Float16)((a[c] - (float)h[c]) * 2048.0f);
+            const float rest = (a[c] - (float)h[c]) * 2048.0f;
+            r[c] = (_Float16)rest;
+            l[c] = (_Float16)((rest - (float)r[c]) * 2048.0f);
         }
         hi[i] = h;
         mid[i] = r;
+        lo[i] = l;
     }
 }
 
-// out[m] = rs[m] (sum of row m's splits + 2^-11 of row M + m's), in split order.
+// out[m] = rs[m] (sum of row m's splits + 2^-11 of row M + m's + 2^-22 of row 2M + m's), in split order.
 __global__ __launch_bounds__(256) void thin_rows_reduce_kernel(const float* __restrict__ raw, int S, int M, int N,
                                                                const float* __restrict__ rs, float* __restrict__ out) {
     const int i = blockIdx.x * 256 + threadIdx.x, N4 = N >> 2;
     if (i >= M * N4) return;
     const int m = i / N4, c = i - m * N4;
     const tf4* r = (const tf4*)raw + (int64_t)m * N4 + c;
-    tf4 a{0.f, 0.f, 0.f, 0.f}, b = a;
-#pragma unroll 4
-    for (int s = 0; s < S; ++s) {
-        a = a + r[(int64_t)s * 2 * M * N4];
-        b = b + r[((int64_t)s * 2 + 1) * M * N4];
+    // eight splits' words on their way before the first is added (one split at a time, the chain of
+    // loads takes three times as long: 22 splits of 8 x 2048 17.6 us)
+    constexpr int G = 8;
+    tf4 sum[3] = {};
+    for (int s0 = 0; s0 < S; s0 += G) {
+        tf4 v[G][3];
+#pragma unroll
+        for (int j = 0; j < G; ++j)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) v[j][q] = r[((int64_t)min(s0 + j, S - 1) * 3 + q) * M * N4];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < G; ++j)
+            if (s0 + j < S)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) sum[q] = sum[q] + v[j][q];
     }
-    ((tf4*)out)[i] = rs[m] * (a + b * (1.0f / 2048.0f));
+    ((tf4*)out)[i] = rs[m] * (sum[0] + (sum[1] + sum[2] * (1.0f / 2048.0f)) * (1.0f / 2048.0f));
 }
 
-template <bool GATEUP>
+template <bool GATEUP, int MAXNT>
 static int thin_dec_launch(int qtype, ThinArgs& a, hipStream_t st) {
     const GemmSplit sp = thin_dec_split(a.N, a.K);
     a.kper = sp.kper;
     const dim3 grid(div_up(a.N, 16 * kThinWaves), 1, sp.ksplit);
     constexpr int R = GATEUP ? 2 : 1;
     switch (qtype) {
-    case PGMOE_Q4_K: PG_LAUNCH((thin_kernel<PGMOE_Q4_K, GATEUP, R, 1>), grid, dim3(kThinThreads), 0, st, a); break;
-    case PGMOE_Q5_K: PG_LAUNCH((thin_kernel<PGMOE_Q5_K, GATEUP, R, 1>), grid, dim3(kThinThreads), 0, st, a); break;
-    case PGMOE_Q6_K: PG_LAUNCH((thin_kernel<PGMOE_Q6_K, GATEUP, R, 1>), grid, dim3(kThinThreads), 0, st, a); break;
+    case PGMOE_Q4_K: PG_LAUNCH((thin_kernel<PGMOE_Q4_K, GATEUP, R, MAXNT, true>), grid, dim3(kThinThreads), 0, st, a); break;
+    case PGMOE_Q5_K: PG_LAUNCH((thin_kernel<PGMOE_Q5_K, GATEUP, R, MAXNT, true>), grid, dim3(kThinThreads), 0, st, a); break;
+    case PGMOE_Q6_K: PG_LAUNCH((thin_kernel<PGMOE_Q6_K, GATEUP, R, MAXNT, true>), grid, dim3(kThinThreads), 0, st, a); break;
     default: return fail(PGMOE_E_UNSUPPORTED, "thin decode: qtype %d", qtype);
     }
     return check_launch("thin decode");
@@ -1004,14 +1022,15 @@ int launch_thin_dense_decode(const Mats& g, const Mats& u, const Mats& d, const 
     ThinArgs a{};
     a.w0 = g.base, a.w1 = u.base, a.N = g.N, a.K = g.K, a.act = x, a.topk = 1, a.P = M;
     a.out = inter, a.act_kind = act, a.raw = raw;
-    int rc = thin_dec_launch<true>(g.qtype, a, st);
+    int rc = thin_dec_launch<true, 1>(g.qtype, a, st);
     if (rc) return rc;
     const int S = thin_dec_split(g.N, g.K).ksplit;
     if ((rc = launch_split_reduce(3, raw, S, M, g.N, nullptr, nullptr, nullptr, inter, st, act))) return rc;
     PG_LAUNCH(thin_rows_kernel, dim3(M), dim3(1024), 0, st, inter, M, g.N, a16, rs);
     ThinArgs b{};
-    b.w0 = d.base, b.N = d.N, b.K = d.K, b.act = a16, b.topk = 1, b.P = 2 * M, b.raw = raw;
-    if ((rc = thin_dec_launch<false>(d.qtype, b, st))) return rc;
+    b.w0 = d.base, b.N = d.N, b.K = d.K, b.act = a16, b.topk = 1, b.P = 3 * M, b.raw = raw;
+    if ((rc = b.P <= 16 ? thin_dec_launch<false, 1>(d.qtype, b, st) : thin_dec_launch<false, 2>(d.qtype, b, st)))
+        return rc;
     PG_LAUNCH(thin_rows_reduce_kernel, dim3(div_up(M * (d.N >> 2), 256)), dim3(256), 0, st, raw,
               thin_dec_split(d.N, d.K).ksplit, M, d.N, rs, out);
     return check_launch("thin decode reduce");

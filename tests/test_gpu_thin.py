@@ -235,3 +235,20 @@ def test_decode_dense_activation(arch):
     a = torch.nn.functional.gelu(g, approximate="tanh") if arch == "gemma3" else torch.nn.functional.silu(g)
     ref = a * torch.from_numpy(up[at, 1].astype(np.float64))
     assert float(((got - ref) / ref).abs().max()) <= (1e-6 if arch == "gemma3" else 6e-7)
+
+
+@pytest.mark.parametrize("M", [5, 8])
+def test_decode_dense_rows_keep_24_bits(M):
+    """Activations of up to 24 bits (whole numbers: SiLU of 10000 is 10000) less their neighbours: every
+    sum is a whole number below 2^24, so the fp32 value of each activation shows in full."""
+    H, I = 2048, 256 * (-(-250000000 // (M * 3 * 2048 * 256)))
+    gate, up, down = np.zeros((I, H), np.int64), np.zeros((I, H), np.int64), np.zeros((H, I), np.int64)
+    i, h = np.arange(I), np.arange(H)
+    gate[:, 0], up[:, 1] = 9 + 2 * (i % 4), 1 + 2 * (i // 4 % 4)
+    a, b = 2 * h % I, (2 * h + 1 + 2 * (h // 16)) % I  # one even, one odd: not the same
+    down[h, a], down[h, b] = 1, -1
+    x = np.zeros((M, H), np.float16)
+    x[:, 0], x[:, 1] = 1021 + 2 * np.arange(M), 135 + 2 * np.arange(M)
+    got = _int_ffn(gate, up, down)(torch.from_numpy(x).to("cuda:0")).cpu().numpy()
+    act = x[:, :1].astype(np.int64) * gate[:, 0] * (x[:, 1:2].astype(np.int64) * up[:, 1])
+    assert act.max() < 2 ** 24 and np.array_equal(got, (act[:, a] - act[:, b]).astype(np.float32))
