@@ -284,10 +284,19 @@ size_t pgmoe_linear_workspace_bytes(const pgmoe_weights* W, int32_t M, int32_t h
  * (round to nearest even).  GGUFQuantLinear.forward (quant_kernels.py:1826-1837 ->
  * exec_w4a16_matmul / exec_w8a16_matmul, :1165-1420) and
  * FusedLinearPack.forward_single_concat (:1895-1898): attention projections, lm_head, the
- * shared expert's fused gate||up.  M <= 8: wavefront GEMV; else the MFMA GEMM (K-quant
- * weights then need their scale plane).  bias: fp32 [N] or NULL.  Host-sync free. */
+ * shared expert's fused gate||up.  M <= 8: wavefront GEMV (3 <= M with 32768 K-quant rows and
+ * more: one MFMA tile on exact weights); else the MFMA products (K-quant weights then need
+ * their scale plane).  bias: fp32 [N] or NULL.  Host-sync free. */
 int pgmoe_linear_forward(const pgmoe_weights* W, const float* bias, const uint16_t* x, int32_t M, void* out,
                          int32_t out_dtype, void* ws, size_t ws_bytes, void* stream);
+
+/* pgmoe_linear_forward for a matrix whose rows are several projections packed (GGUFQuantLinear.fuse,
+ * quant_kernels.py:1635): member_rows is the row count of the smallest one.  For M <= 8 the
+ * kernel is chosen by it, as pgmoe_linear_forward chooses by a matrix's own rows, so that a
+ * projection's outputs are the same bits packed and alone (unless members lie on both sides
+ * of that choice: the larger ones then run as the smallest does).  Same workspace. */
+int pgmoe_linear_forward_packed(const pgmoe_weights* W, int32_t member_rows, const float* bias, const uint16_t* x,
+                                int32_t M, void* out, int32_t out_dtype, void* ws, size_t ws_bytes, void* stream);
 
 /* Rows rows[0..n) of W dequantised: out[n, K] (PGMOE_DT_F32 or PGMOE_DT_F16); values as
  * the ggml block definitions give them with fp32 products; an id outside [0, N) gives a

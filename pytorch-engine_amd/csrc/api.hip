@@ -604,10 +604,17 @@ size_t pgmoe_linear_workspace_bytes(const pgmoe_weights* W, int32_t M, int32_t h
 
 int pgmoe_linear_forward(const pgmoe_weights* W, const float* bias, const uint16_t* x, int32_t M, void* out,
                          int32_t out_dtype, void* ws, size_t ws_bytes, void* stream) {
+    return pgmoe_linear_forward_packed(W, W ? W->n_rows : 0, bias, x, M, out, out_dtype, ws, ws_bytes, stream);
+}
+
+int pgmoe_linear_forward_packed(const pgmoe_weights* W, int32_t member_rows, const float* bias, const uint16_t* x,
+                                int32_t M, void* out, int32_t out_dtype, void* ws, size_t ws_bytes, void* stream) {
     Mats w;
     int rc = check_weights(W, "linear", &w);
     if (rc) return rc;
     if (w.n_mats != 1) return fail(PGMOE_E_INVALID, "linear: one matrix (n_mats = 1), got %d", w.n_mats);
+    if (member_rows < 1 || member_rows > w.N)
+        return fail(PGMOE_E_INVALID, "linear: %d rows of a member outside [1, %d]", member_rows, w.N);
     if (M < 0) return fail(PGMOE_E_INVALID, "negative token count");
     if (out_dtype != PGMOE_DT_F32 && out_dtype != PGMOE_DT_F16)
         return fail(PGMOE_E_UNSUPPORTED, "linear: output dtype %d (F32=0, F16=1)", out_dtype);
@@ -617,7 +624,8 @@ int pgmoe_linear_forward(const pgmoe_weights* W, const float* bias, const uint16
         return fail(PGMOE_E_INVALID, "linear: x must be 16-byte, ws 256-byte, out 4-byte aligned");
     if (w.qtype != PGMOE_Q8_0 && w.qtype != PGMOE_F16 && !w.scales && !linear_gemv_fits(M, w.K))
         return fail(PGMOE_E_INVALID, "linear: K-quant weights need their scale plane for %d tokens", M);
-    return launch_linear(w, bias, x, M, out, out_dtype == PGMOE_DT_F16, (uint8_t*)ws, ws_bytes, as_stream(stream));
+    return launch_linear(w, member_rows, bias, x, M, out, out_dtype == PGMOE_DT_F16, (uint8_t*)ws, ws_bytes,
+                         as_stream(stream));
 }
 
 int pgmoe_dequant_rows(const pgmoe_weights* W, const int32_t* rows, int32_t n, void* out, int32_t out_dtype,

@@ -120,9 +120,10 @@ int launch_dec_linear(const Mats& w, const uint16_t* x, int M, const float* bias
 // Whether the decode GEMV can stage M rows of K inputs (the linear's M <= 8 path).
 bool linear_gemv_fits(int M, int K);
 // The quantized linear (linear.hip): out[M, N] = x . W^T (+ bias), fp32 or fp16; ws of
-// linear_ws_bytes(w, M, bias || out_f16) bytes (none on the GEMV path).
+// linear_ws_bytes(w, M, bias || out_f16) bytes (none on the GEMV path).  member_rows: rows of the
+// smallest projection packed in w (w.N: one alone).
 size_t linear_ws_bytes(const Mats& w, int M, bool staged);
-int launch_linear(const Mats& w, const float* bias, const uint16_t* x, int M, void* out, int out_f16, uint8_t* ws,
+int launch_linear(const Mats& w, int member_rows, const float* bias, const uint16_t* x, int M, void* out, int out_f16, uint8_t* ws,
                   size_t ws_bytes, hipStream_t st);
 // Rows rows[0..n) of w decoded to out [n, K] (fp32, or fp16 with out_f16).
 int launch_dequant_rows(const Mats& w, const int32_t* rows, int n, void* out, int out_f16, hipStream_t st);
@@ -182,7 +183,7 @@ int launch_thin_down(const Mats& d, const uint16_t* a16, const float* rs, int M,
 int launch_thin_linear(const Mats& w, const uint16_t* x, int M, const float* bias, void* out, int out_f16, float* raw,
                        hipStream_t st);
 // A decode linear (M <= 8) on a thin tile, where thin_takes_decode: exact weights, fp32 sums.
-bool thin_takes_decode(int qtype, int M, int N, int K);
+bool thin_takes_decode(const Mats& w, int member_rows, int M);
 int launch_thin_decode(const Mats& w, const uint16_t* x, int M, const float* bias, void* out, int out_f16,
                        hipStream_t st);
 // A decode FFN on thin tiles (a16: 3 M rows of I halves; rs: M; raw: thin_dec_raw_bytes).

@@ -135,10 +135,10 @@ size_t linear_ws_bytes(const Mats& w, int M, bool staged) {
     return n + al(gemm_split_bytes_upto(M, 1, w.N, w.K, false));  // split-K partial sums (any batch up to M)
 }
 
-int launch_linear(const Mats& w, const float* bias, const uint16_t* x, int M, void* out, int out_f16, uint8_t* ws,
-                  size_t ws_bytes, hipStream_t st) {
+int launch_linear(const Mats& w, int member_rows, const float* bias, const uint16_t* x, int M, void* out, int out_f16,
+                  uint8_t* ws, size_t ws_bytes, hipStream_t st) {
     if (M == 0) return PGMOE_OK;
-    if (linear_gemv(M, w.K) && thin_takes_decode(w.qtype, M, w.N, w.K))
+    if (linear_gemv(M, w.K) && thin_takes_decode(w, member_rows, M))
         return launch_thin_decode(w, x, M, bias, out, out_f16, st);
     if (linear_gemv(M, w.K)) return launch_dec_linear(w, x, M, bias, out, out_f16, st);
     const bool staged = bias || out_f16;

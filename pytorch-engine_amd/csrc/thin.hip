@@ -880,12 +880,12 @@ int launch_thin_down(const Mats& d, const uint16_t* a16, const float* rs, int M,
 // weight once but spends a dot2 and two LDS bytes on it for each token, so 8 tokens cost it twice
 // the weights' time; here 16 rows of MFMA cost what one does.  2048 x 151936, us GEMV -> here:
 // Q6_K 3 rows 70 -> 62, 8 rows 121 -> 64; Q4_K 56 -> 45, 103 -> 46; Q5_K 62 -> 53, 107 -> 55 (two
-// rows: Q6_K 60 -> 62).  Q8_0's d q is no fp16 value, so it stays there.  K is not split, so
-// that outputs depend on no other rows of a pack: from a block a CU on.
+// rows: Q6_K 60 -> 62).  Q8_0's d q is no fp16 value, so it stays there.  K is not split: from a
+// block a CU on.  The rule looks at the smallest projection of a pack, whose rows then have the
+// same bits alone and packed (gate || up of 20480 rows each stays on the GEMV, as each does).
 static bool thin_exact(int qtype) { return qtype == PGMOE_Q4_K || qtype == PGMOE_Q5_K || qtype == PGMOE_Q6_K; }
-bool thin_takes_decode(int qtype, int M, int N, int K) {
-    return thin_exact(qtype) && M > 2 && N >= 32768 && N % 4 == 0 &&
-           (int64_t)M * K < ((int64_t)1 << 31);
+bool thin_takes_decode(const Mats& w, int member_rows, int M) {
+    return thin_exact(w.qtype) && M > 2 && member_rows >= 32768 && (int64_t)M * w.K < ((int64_t)1 << 31);
 }
 
 int launch_thin_decode(const Mats& w, const uint16_t* x, int M, const float* bias, void* out, int out_f16,

@@ -112,6 +112,8 @@ def lib() -> ctypes.CDLL:
     L.pgmoe_linear_workspace_bytes.restype = ctypes.c_size_t
     L.pgmoe_linear_workspace_bytes.argtypes = [ctypes.POINTER(Weights), _I32, _I32, _I32]
     L.pgmoe_linear_forward.argtypes = [ctypes.POINTER(Weights), _P, _P, _I32, _P, _I32, _P, ctypes.c_size_t, _P]
+    L.pgmoe_linear_forward_packed.argtypes = [ctypes.POINTER(Weights), _I32, _P, _P, _I32, _P, _I32, _P,
+                                              ctypes.c_size_t, _P]
     L.pgmoe_dequant_rows.argtypes = [ctypes.POINTER(Weights), _P, _I32, _P, _I32, _P]
     L.pgmoe_add_rmsnorm.argtypes = [_P, _I32, _P, _I32, _P, _I32, _I32, ctypes.c_float, _P, _P, _I32, _P]
     L.pgmoe_moe_forward_noalloc.argtypes = [ctypes.POINTER(Layer), _P, _I32, _P, _P]
@@ -132,8 +134,8 @@ def lib() -> ctypes.CDLL:
                "pgmoe_expert_down", "pgmoe_combine", "pgmoe_relayout_weights", "pgmoe_relayout_weights_padded",
                "pgmoe_build_scale_plane",
                "pgmoe_dense_forward", "pgmoe_moe_routing", "pgmoe_moe_status", "pgmoe_moe_forward_noalloc",
-               "pgmoe_add_rmsnorm", "pgmoe_linear_forward", "pgmoe_dequant_rows", "pgmoe_requant_w4",
-               "pgmoe_requant_w8_f16"):
+               "pgmoe_add_rmsnorm", "pgmoe_linear_forward", "pgmoe_linear_forward_packed", "pgmoe_dequant_rows",
+               "pgmoe_requant_w4", "pgmoe_requant_w8_f16"):
         getattr(L, fn).restype = ctypes.c_int
     ver = L.pgmoe_abi_version()
     if ver != ABI_VERSION:
@@ -157,6 +159,7 @@ EXPORTS = (
     "pgmoe_dense_workspace_bytes", "pgmoe_dense_forward", "pgmoe_moe_routing", "pgmoe_moe_status",
     "pgmoe_moe_forward_noalloc", "pgmoe_add_rmsnorm", "pgmoe_linear_workspace_bytes", "pgmoe_linear_forward",
     "pgmoe_dequant_rows", "pgmoe_relayout_weights_padded", "pgmoe_requant_w4", "pgmoe_requant_w8_f16",
+    "pgmoe_linear_forward_packed",
 )
 
 STATUS_SPIN_TIMEOUT = 1  # PGMOE_STATUS_SPIN_TIMEOUT

@@ -1,4 +1,4 @@
-"""GGUFQuantLinear / FusedLinearPack on the HIP kernels (pgmoe_linear_forward).
+"""GGUFQuantLinear / FusedLinearPack on the HIP kernels (pgmoe_linear_forward_packed).
 
 Drop-ins for the reference's quantized linear (pygguf_engine/quant_kernels.py:1604-1915),
 the module behind its attention projections, lm_head, embedding table and the shared
@@ -11,7 +11,8 @@ expert's fused gate||up:
     FusedLinearPack(linears).forward(x) / .forward_single_concat(x)
 
 The weights stay in GGUF block form on the device (the 64-row tile layout of the MoE
-experts); M <= 8 tokens run the wavefront GEMV, more run the MFMA GEMM.  Unquantised
+experts); M <= 8 tokens run the wavefront GEMV (3 .. 8 of them on a K-quant output head one
+MFMA tile), more run the MFMA products.  Unquantised
 weights (F16 / F32 / BF16, the reference's "fp16" mode) run torch's fp16 F.linear on the
 device, as in the reference.  There is no CPU path: quantised formats without a kernel,
 rows whose width is not a multiple of 256, and CPU devices raise.  The reference's
@@ -49,6 +50,7 @@ class GGUFQuantLinear(nn.Module):
         self.mode = mode  # "w4" / "w8" (quantised, by the reference's naming) or "fp16"
         self.in_features = int(in_features)
         self.out_features = int(out_features)
+        self.member_rows = int(out_features)  # of the smallest projection fused in this one
         self.gguf_qtype = gguf_qtype
         dev = torch.device(device if device is not None else (weight.device if weight is not None else "cuda"))
         if dev.type != "cuda":
@@ -128,7 +130,9 @@ class GGUFQuantLinear(nn.Module):
             w = torch.cat([lin.weight for lin in linears], dim=0)
             return cls("fp16", first.in_features, total, weight=w, bias=bias, device=first.device)
         raw = np.concatenate([np.asarray(lin._raw).reshape(-1) for lin in linears])
-        return cls(first.mode, first.in_features, total, first.gguf_qtype, raw=raw, bias=bias, device=first.device)
+        fused = cls(first.mode, first.in_features, total, first.gguf_qtype, raw=raw, bias=bias, device=first.device)
+        fused.member_rows = min(lin.member_rows for lin in linears)
+        return fused
 
     # ------------------------------------------------------------------ compute
     def forward(self, x: torch.Tensor) -> torch.Tensor:
@@ -151,9 +155,10 @@ class GGUFQuantLinear(nn.Module):
             stream = torch.cuda.current_stream(self.device).cuda_stream
             n = int(lib().pgmoe_linear_workspace_bytes(self._w, M, int(self.bias is not None), _OUT[odt]))
             ws = self._ws.get(max(n, 1), stream)
-            check(lib().pgmoe_linear_forward(self._w, None if self.bias is None else self.bias.data_ptr(),
-                                             xh.data_ptr(), M, out.data_ptr(), _OUT[odt], ws.data_ptr(), ws.numel(),
-                                             stream), "pgmoe_linear_forward")
+            check(lib().pgmoe_linear_forward_packed(self._w, self.member_rows,
+                                                    None if self.bias is None else self.bias.data_ptr(),
+                                                    xh.data_ptr(), M, out.data_ptr(), _OUT[odt], ws.data_ptr(),
+                                                    ws.numel(), stream), "pgmoe_linear_forward_packed")
         if odt != x.dtype:
             out = out.to(x.dtype)
         return out.reshape(*orig_shape[:-1], self.out_features)

@@ -330,3 +330,14 @@ def test_f16_weight_sizes_and_planes():
     assert L.pgmoe_weight_bytes(1, 64, 320) == -1
     from pgmoe import ops
     assert ops.device_qtype(0) == ops.device_qtype(30) == ops.device_qtype(1) == 1
+
+
+def test_packed_linear_checks_the_member_rows():
+    L = _lib.lib()
+    lin = _lib.Weights(12, 1024, 512, 1, 0x100000, 0)
+    for rows in (0, -1, 1025):
+        assert L.pgmoe_linear_forward_packed(lin, rows, None, 0x1000, 4, 0x2000, 0, None, 0, None) == -1
+        assert b"member" in L.pgmoe_last_error()
+    assert L.pgmoe_linear_forward_packed(lin, 1024, None, 0x1000, 0, 0x2000, 0, None, 0, None) == 0
+    assert L.pgmoe_linear_forward_packed(None, 1, None, 0x1000, 4, 0x2000, 0, None, 0, None) == -1
+    assert L.pgmoe_linear_forward(None, None, 0x1000, 4, 0x2000, 0, None, 0, None) == -1

@@ -252,3 +252,20 @@ def test_decode_dense_rows_keep_24_bits(M):
     got = _int_ffn(gate, up, down)(torch.from_numpy(x).to("cuda:0")).cpu().numpy()
     act = x[:, :1].astype(np.int64) * gate[:, 0] * (x[:, 1:2].astype(np.int64) * up[:, 1])
     assert act.max() < 2 ** 24 and np.array_equal(got, (act[:, a] - act[:, b]).astype(np.float32))
+
+
+@pytest.mark.parametrize("qt", [Q4_K, Q6_K])
+@pytest.mark.parametrize("rows", [(16384, 16420), (32769, 32768)])
+def test_packed_projections_equal_separate_ones(qt, rows):
+    """Up to 8 tokens a projection has the same bits packed and alone, also where only the pack, or
+    each member too, has the rows of an output head."""
+    from pgmoe import FusedLinearPack, GGUFQuantLinear
+    dev = torch.device("cuda", 0)
+    rng = np.random.default_rng(sum(rows) + qt)
+    lins = [GGUFQuantLinear("w8", 512, n, qt, raw=random_blocks(rng, qt, n, 512, 0.01), device=dev) for n in rows]
+    pack = FusedLinearPack(lins)
+    for M in (1, 2, 3, 5, 8):
+        log(f"packed qt={qt} rows={rows} M={M}")
+        x = torch.from_numpy(rng.standard_normal((M, 512)).astype(np.float16)).to(dev)
+        for got, lin in zip(pack(x.float()), lins):
+            assert torch.equal(got, lin(x.float()))
