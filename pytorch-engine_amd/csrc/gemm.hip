@@ -142,11 +142,25 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 typedef _Float16 gh2 __attribute__((ext_vector_type(2)));
 
 // w = a * code + c2 as fp16 for 8 codes given as fp16 (1024 + code) pairs (c2 = c - 1024a
-// folded by the caller: one fp32 FMA per weight, one rounding to fp16).  As two v_fma_mix_f32
-// and a v_cvt_pk_f16_f32 a pair (4 cycles each): v_fma_mixlo / mixhi_f16, which the compiler
-// took for a quarter of the pairs, need 8 each.  Qwen3 skewed prompt of 4096 tokens -0.7 %, a
-// 1500-token FFN (H = 4096, I = 12288) -0.7 %.
+// folded by the caller: one fp32 FMA per weight, one rounding to fp16).  CVT: as two
+// v_fma_mix_f32 and a v_cvt_pk_f16_f32 a pair (4 cycles each; Qwen3 skewed prompt of 4096 tokens
+// -0.7 %, a 1500-token FFN (H = 4096, I = 12288) -0.7 %).  Without it the compiler takes
+// v_fma_mixlo / mixhi_f16 (8 cycles each) for a quarter of the pairs, fewer instructions: better
+// where a wave has up to three slices of rows to multiply them with and the decode's latency
+// shows (96 rows: 2048 x 151936 Q4_K 140.5 -> 136.0 us, 8192 x 57344 Q4_K 167.0 -> 162.5; 120
+// rows alike).  Same bits.
+template <bool CVT>
 __device__ __forceinline__ gh8 deq8(const uint32_t (&m)[4], float a, float c) {
+    if constexpr (!CVT) {
+        gh8 r;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const gh2 h = __builtin_bit_cast(gh2, m[k]);
+            r[2 * k] = (_Float16)__builtin_fmaf((float)h.x, a, c);
+            r[2 * k + 1] = (_Float16)__builtin_fmaf((float)h.y, a, c);
+        }
+        return r;
+    }
     typedef float f2 __attribute__((ext_vector_type(2)));
     gh2 r[4];
 #pragma unroll
@@ -198,12 +212,13 @@ template <> struct GCol<PGMOE_Q4_K> {
         a[1] = sv.z;
         c[1] = sv.w;
     }
+    template <bool CVT>
     __device__ __forceinline__ gh8 group(int g) const {
         const u32x2 s = q[g & 1];
         const int sh = 4 * (g >> 1);
         uint32_t m[4];
         magic8((s.x >> sh) & 0x0f0f0f0fu, (s.y >> sh) & 0x0f0f0f0fu, m);
-        return deq8(m, a[g >> 1], c[g >> 1]);
+        return deq8<CVT>(m, a[g >> 1], c[g >> 1]);
     }
 };
 
@@ -229,6 +244,7 @@ template <> struct GCol<PGMOE_Q5_K> {
         a[1] = sv.z;
         c[1] = sv.w;
     }
+    template <bool CVT>
     __device__ __forceinline__ gh8 group(int g) const {
         // elements 16(g & 1) + 8h + [0, 8) of sub-block 2(u%4) + (g >> 1): quads 4(g & 1) + 2h, + 1
         const u32x2 s = q[g & 1];
@@ -238,7 +254,7 @@ template <> struct GCol<PGMOE_Q5_K> {
         const uint32_t c1 = ((s.y >> sh) & 0x0f0f0f0fu) | (((w >> (hb + 1)) & 0x01010101u) << 4);
         uint32_t m[4];
         magic8(c0, c1, m);
-        return deq8(m, a[g >> 1], c[g >> 1]);
+        return deq8<CVT>(m, a[g >> 1], c[g >> 1]);
     }
 };
 
@@ -259,6 +275,7 @@ template <> struct GCol<PGMOE_Q6_K> {
         a[2] = sv.z;
         a[3] = sv.w;
     }
+    template <bool CVT>
     __device__ __forceinline__ gh8 group(int g) const {
         const u32x2 l = q[g & 1], hq = q[2];
         const int sh = 4 * (g >> 1), hs = 2 * g;
@@ -266,7 +283,7 @@ template <> struct GCol<PGMOE_Q6_K> {
         const uint32_t c1 = ((l.y >> sh) & 0x0f0f0f0fu) | (((hq.y >> hs) & 0x03030303u) << 4);
         uint32_t m[4];
         magic8(c0, c1, m);
-        return deq8(m, a[g], -1056.0f * a[g]);  // (1024 + q6) a - 1056 a = (q6 - 32) a
+        return deq8<CVT>(m, a[g], -1056.0f * a[g]);  // (1024 + q6) a - 1056 a = (q6 - 32) a
     }
 };
 
@@ -280,6 +297,7 @@ template <> struct GCol<PGMOE_Q8_0> {
         dw = *(const uint32_t*)(base + 4 * 1024 + 4 * (u & 3));
     }
     __device__ __forceinline__ void prep(int) {}
+    template <bool CVT>
     __device__ __forceinline__ gh8 group(int g) const {
         const u32x2 s = q[g];
         uint32_t m[4];
@@ -305,6 +323,7 @@ template <> struct GCol<PGMOE_F16> {
         for (int g = 0; g < 4; ++g) c[g] = *(const gu4*)(base + (2 * g + h) * 1024);
     }
     __device__ __forceinline__ void prep(int u) {}
+    template <bool CVT>
     __device__ __forceinline__ gh8 group(int g) const { return __builtin_bit_cast(gh8, c[g]); }
 };
 
@@ -382,7 +401,7 @@ __device__ __forceinline__ void gemm_loop(const uint8_t* smem, int units, const 
 #pragma unroll
         for (int i = 0; i < NI; ++i) a[i] = *(const gh8*)(p + 4096 * i);
 #pragma unroll
-        for (int j = 0; j < CT; ++j) b[j] = col[j].group(g);
+        for (int j = 0; j < CT; ++j) b[j] = col[j].template group<(NI > 3)>(g);
     };
     const std::integral_constant<int, AC> ac;
 #pragma unroll
