@@ -273,7 +273,7 @@ int pgmoe_dense_forward(const pgmoe_dense* D, const uint16_t* x, int32_t M, floa
                                            out, nullptr, 0, st);
         return launch_dec_down_ident(d, WS(float, inter), WS(float, isum), M, out, st);
     }
-    const bool tg = thin_takes(g.qtype, M, 1, g.N, g.K, true), td = thin_takes(d.qtype, M, 1, d.N, d.K, false);
+    const bool tg = thin_takes(g.qtype, M, g.N, g.K, true), td = thin_takes(d.qtype, M, d.N, d.K, false);
     if ((!tg || !td) &&
         (rc = launch_identity_dispatch(M, gemm_tile_rows(), WS(int32_t, offsets), WS(int32_t, perm), WS(int32_t, inv),
                                        WS(int32_t, active), WS(int32_t, nact), WS(int32_t, tile_off), WS(float, w),
@@ -513,8 +513,7 @@ static int moe_forward_impl(const pgmoe_layer* L, const LayerMats& lm, const Lay
     if ((rc = launch_router_logits(x, L->router_w, L->router_bias, M, H, E, WS(float, logits), st))) return rc;
     if ((rc = launch_topk(WS(float, logits), M, E, K, L->norm_topk, WS(int32_t, idx), WS(float, w), st))) return rc;
     const int64_t P = (int64_t)M * K;
-    if (thin_takes(lm.gate.qtype, P, E, lm.gate.N, lm.gate.K, true) &&
-        thin_takes(lm.down.qtype, P, E, lm.down.N, lm.down.K, false)) {  // few pairs an expert
+    if (thin_takes_moe(lm.gate, lm.down, M, K)) {  // few pairs an expert
         if ((rc = launch_dispatch(WS(int32_t, idx), M, K, E, thin_tile_rows(), WS(int32_t, offsets), WS(int32_t, perm),
                                   WS(int32_t, inv), WS(int32_t, active), WS(int32_t, nact), WS(int32_t, tile_off), st,
                                   WS(int32_t, dcounts))) ||
@@ -543,8 +542,8 @@ static int moe_forward_impl(const pgmoe_layer* L, const LayerMats& lm, const Lay
     const float* shared = nullptr;
     const float* shared_logit = nullptr;
     if (L->has_shared) {
-        const bool tg = thin_takes(lm.sg.qtype, M, 1, lm.sg.N, lm.sg.K, true);
-        const bool td = thin_takes(lm.sd.qtype, M, 1, lm.sd.N, lm.sd.K, false);
+        const bool tg = thin_takes(lm.sg.qtype, M, lm.sg.N, lm.sg.K, true);
+        const bool td = thin_takes(lm.sd.qtype, M, lm.sd.N, lm.sd.K, false);
         if ((!tg || !td) &&
             (rc = launch_identity_dispatch(M, gemm_tile_rows(), WS(int32_t, s_offsets), WS(int32_t, s_perm),
                                            WS(int32_t, s_inv), WS(int32_t, s_active), WS(int32_t, s_nact),

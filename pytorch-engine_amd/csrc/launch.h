@@ -173,7 +173,8 @@ int launch_split_reduce(int kind, const float* raw, int S, int64_t P, int N, con
 // arguments as the grouped GEMMs (tile_off counts thin tiles).  offsets, perm, tile_off and
 // topk_w null: one matrix, pair p is row p with weight 1.  raw: split-K scratch of the
 // grouped GEMM's size, or null.
-bool thin_takes(int qtype, int64_t P, int E, int N, int K, bool gateup);
+bool thin_takes(int qtype, int64_t P, int N, int K, bool gateup);
+bool thin_takes_moe(const Mats& g, const Mats& d, int M, int topk);
 int thin_tile_rows();
 int launch_thin_gateup(const Mats& g, const Mats& u, const uint16_t* x, int M, int topk, const int32_t* offsets,
                        const int32_t* perm, const int32_t* tile_off, float* inter, hipStream_t st, float* raw, int act);

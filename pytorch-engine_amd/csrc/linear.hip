@@ -160,7 +160,7 @@ int launch_linear(const Mats& w, int member_rows, const float* bias, const uint1
     float* prod = staged ? (float*)take((size_t)M * w.N * 4) : (float*)out;
     const size_t rb = gemm_split_bytes(M, 1, w.N, w.K, false);
     float* raw = rb ? (float*)take(rb) : nullptr;
-    if (thin_takes(w.qtype, M, 1, w.N, w.K, false)) return launch_thin_linear(w, x, M, bias, out, out_f16, raw, st);
+    if (thin_takes(w.qtype, M, w.N, w.K, false)) return launch_thin_linear(w, x, M, bias, out, out_f16, raw, st);
     int rc = launch_identity_dispatch(M, gemm_tile_rows(), offsets, perm, inv, active, nact, tile_off, ones, st);
     if (rc) return rc;
     // the down GEMM's epilogue scales row p by rs[p] * topk_w[perm[p]]: both 1 here

@@ -766,26 +766,48 @@ __global__ __launch_bounds__(kThinThreads, 4) void thin_kernel(const ThinArgs A)
 constexpr int kThinTile = 32;
 int thin_tile_rows() { return kThinTile; }
 
-// Whether the product of P pairs with E matrices [N, K] takes thin tiles.  Each tile decodes
-// its weights again, so the 256-row tiles win once an expert's pairs fill a few of them:
-//   grouped: up to 40 pairs an expert (Qwen3 shape, whole layer: 512 tokens = 32 an expert 206
-//     -> 188 us, 768 = 48 225 -> 235; Mixtral 128 = 32 351 -> 296, 256 = 64 406 -> 447), up to
-//     24 where the 256-row tiles read no scale plane either (Q8_0, F16; Qwen2 shape: 20 an
-//     expert 600 -> 559, 31 657 -> 695);
-//   one matrix, by the weights decoded in all (work): up to 850 M for 256 rows, where the
-//     256-row tiles have one M tile (H = 4096, I = 12288 FFN: 256 rows 162 -> 152 us; Qwen2's
-//     shared expert, 250 rows and 1174 M: 686 -> 705), above that up to 450 M while those tiles
-//     leave most CUs idle (4096 x 6144 Q4_K linear, 512 rows: 77 -> 53; the FFN's down product,
-//     384 rows and 604 M, loses 13 us; above 512 rows up to 150 M: 2048 x 1024 Q8_0, 1024 rows 35
-//     -> 17, but an I = 5632 down product of 1024 rows and 369 M loses 6); fp16 weights, which take the 256-row tiles without any
-//     decode, one tile (I = 5632 FFN: 32 rows 42 -> 36 us, 64 rows 46 -> 49).
-bool thin_takes(int qtype, int64_t P, int E, int N, int K, bool gateup) {
+// Whether the product of P rows with one matrix [N, K] takes thin tiles.  Each tile decodes its weights
+// again (about 7 M a us), so the 256-row tiles win once the rows fill a few of them; work: the weights
+// decoded in all.  Cold weights, us 256-row tiles -> thin tiles:
+//   up to 256 rows, where the 256-row tiles have one M tile: gate / up (two row tiles a wave) up to
+//     510 M (H = 4096, I = 12288 FFN, Q4_K: 160 rows 133 -> 112, 192 rows = 604 M 147 -> 147, 256
+//     172 -> 180; Q5_K 192 150 -> 173), else up to 850 M (28672 x 4096 Q4_K, 192 rows and 704 M 107
+//     -> 101) and 4 MB of rows, an XCD's L2 (a down product of 20480 inputs and Q4_K, 128 rows,
+//     loses 3 us of 144, one of 12288 and 192 rows 2 of 150; 4096 x 28672 Q5_K: 16 rows 49 -> 26, 64 54
+//     -> 51, 96 59 -> 71);
+//   above, up to 450 M while those tiles leave most CUs idle (4096 x 6144 Q4_K linear, 512 rows: 86 ->
+//     57; 512 rows and more up to 150 M: 2048 x 1024 Q8_0, 1024 rows 41 -> 20, but an I = 5632 down
+//     product of 1024 rows and 369 M loses 6);
+//   fp16 weights, which the 256-row tiles take without any decode, one tile (I = 5632 FFN: 32 rows 59 ->
+//     53, 64 rows 62 -> 64).
+bool thin_takes(int qtype, int64_t P, int N, int K, bool gateup) {
     if (N % 4 || P * K >= ((int64_t)1 << 31)) return false;  // split sums of four; 32-bit row offsets
-    if (E > 1) return P <= (int64_t)E * (qtype == PGMOE_Q8_0 || qtype == PGMOE_F16 ? 24 : 40);
     if (qtype == PGMOE_F16) return P <= kThinTile;
     const int64_t work = (int64_t)div_up(P, kThinTile) * N * K * (gateup ? 2 : 1);
-    if (P <= 256) return work <= 850000000;
+    if (P <= 256) return gateup ? work <= 510000000 : work <= 850000000 && P * K <= 1 << 21;
     return work <= (P <= 512 ? 450000000 : 150000000) && (int64_t)div_up(P, 256) * div_up(N, gateup ? 128 : 256) <= 96;
+}
+
+// Whether an MoE layer's products take thin tiles, for every routing of M tokens to topk experts each
+// (the device's alone to know).  Cold weights, us 256-row tiles -> thin tiles, a layer:
+//   all tokens on the same experts, each then M rows: while the gate / up weights decoded, times the
+//     K splits that keep the 256-row tiles' CUs busy on so few experts, are up to 475 M (Mixtral
+//     shape 64 tokens = 470 M 135 -> 131, 72 150 -> 171, 128 168 -> 212; Qwen2 96 = 440 M 137 -> 132,
+//     100 150 -> 154, 192 193 -> 207; Qwen3 448 147 -> 127; 8 experts of 6144 inputs, two splits, 64
+//     = 403 M 93 -> 84, 96 103 -> 115);
+//   even and Zipf-like: up to 30 pairs an expert (Qwen3 448 tokens = 28: 213 -> 167 and 149 -> 137, 512
+//     = 32: 218 -> 184 and 146 -> 150), 24 where the 256-row tiles read no scale plane either (Q8_0;
+//     Qwen2 96 = 12: 411 -> 367 and 256 -> 229), and 2 for F16, which they take as it is stored (H =
+//     2048, I = 768, 128 experts: 32 tokens 310 -> 291, 64 326 -> 328; I = 6144, 8: 16 319 -> 329).
+bool thin_takes_moe(const Mats& g, const Mats& d, int M, int topk) {
+    const int64_t P = (int64_t)M * topk;
+    const int E = g.n_mats;
+    if (E == 1) return thin_takes(g.qtype, P, g.N, g.K, true) && thin_takes(d.qtype, P, d.N, d.K, false);
+    if (g.N % 4 || d.N % 4 || P * std::max(g.K, d.K) >= ((int64_t)1 << 31)) return false;
+    for (const Mats* m : {&g, &d})
+        if (P > (int64_t)E * (m->qtype == PGMOE_F16 ? 2 : m->qtype == PGMOE_Q8_0 ? 24 : 30)) return false;
+    return (int64_t)std::min(topk, E) * div_up(M, kThinTile) * g.N * g.K * 2 * gemm_split(P, E, g.N, g.K, true).ksplit <=
+           475000000;
 }
 
 // Splits of K, cut at super-block boundaries: the count with the least estimated time, rounds

@@ -80,7 +80,8 @@ def test_decode_linear_of_many_rows(qt, K):
                                           (F16, F16)])
 def test_layer_tiles(gate_up, down):
     """A skewed router: with M tokens the first expert holds about M pairs (tiles of 32 and a
-    remainder), the others few or none; M = 160 / 161 lie on both sides of 40 pairs an expert."""
+    remainder), the others few or none; M = 120 / 121 lie on both sides of 30 pairs an expert, 96 / 97 of
+    24 (Q8_0; F16 takes the 256-row tiles from 9 tokens on)."""
     spec = LayerSpec("thin", 768, 8, 2, 512, (gate_up, gate_up, down), shared_inter=256,
                      shared_qtypes=(gate_up, gate_up, down), shared_gate=True)
     # float weights at their own scale: at 0.01 (2e-4) the SwiGLU rows, near 1e-6, fall among
@@ -89,7 +90,7 @@ def test_layer_tiles(gate_up, down):
     bias = np.array([6, 1, 0, 0, -1, -1, -2, -8], np.float32)
     mod.set_router_bias(torch.from_numpy(bias))
     ol = oracle.OracleLayer.from_gguf(lay.gguf, lay.config, router_bias=bias)
-    for M in (9, 16, 33, 47, 96, 97, 160, 161):
+    for M in (9, 16, 33, 47, 96, 97, 120, 121, 160, 161):
         log(f"thin layer {gate_up}/{down} M={M}")
         x = lay.draw_x(M)
         got = mod(torch.from_numpy(x).to("cuda:0")).cpu().numpy()
@@ -123,8 +124,8 @@ def test_decode_dense_on_thin_tiles(gate_up, down, H, I):
 
 
 def test_dense_sides_of_the_rule_and_replays():
-    """Both products on thin tiles, only the down one, and neither; a captured forward on thin
-    tiles equals the eager one at every replay."""
+    """Both products on thin tiles (9 tokens), only gate / up (100, 256), only the down one (257) and
+    neither (600); a captured forward on thin tiles equals the eager one at every replay."""
     from pgmoe import HipDenseMLP
     dev = torch.device("cuda", 0)
     lay = SyntheticDense(DenseSpec("thin", 1024, 25600, (Q4_K, Q4_K, Q6_K)), seed=2, scale=0.01)
@@ -269,3 +270,37 @@ def test_packed_projections_equal_separate_ones(qt, rows):
         x = torch.from_numpy(rng.standard_normal((M, 512)).astype(np.float16)).to(dev)
         for got, lin in zip(pack(x.float()), lins):
             assert torch.equal(got, lin(x.float()))
+
+
+def test_layer_on_few_experts_at_both_sides_of_the_rule():
+    """Every token on the same two experts: 96 tokens take thin tiles (three an expert), 97 not."""
+    spec = LayerSpec("conc", 4096, 8, 2, 8192, (Q4_K, Q4_K, Q4_K))
+    lay, ol, mod = build_pair(spec, seed=6, scale=0.01)
+    bias = np.array([0, 40, 0, 0, 0, 0, 40, 0], np.float32)
+    mod.set_router_bias(torch.from_numpy(bias))
+    ol = oracle.OracleLayer.from_gguf(lay.gguf, lay.config, router_bias=bias)
+    for M in (64, 96, 97):
+        log(f"thin layer on two experts M={M}")
+        x = lay.draw_x(M)
+        got = mod(torch.from_numpy(x).to("cuda:0")).cpu().numpy()
+        _, idx, w = ol.route(x)
+        assert set(idx.reshape(-1).tolist()) == {1, 6}
+        check_forward_routing(mod, M, idx, w)
+        toks = np.array([0, 31, 32, M - 1])
+        check_layer_output(got[toks], ol.forward_tokens(x[toks], idx[toks], w[toks]))
+
+
+def test_layer_tiles_of_fp16_experts():
+    """fp16 experts take thin tiles up to two pairs an expert (48 tokens here)."""
+    spec = LayerSpec("thin16", 512, 48, 2, 256, (F16, F16, F16))
+    lay, ol, mod = build_pair(spec, seed=7)
+    bias = np.where(np.arange(48) == 5, 3.0, 0.0).astype(np.float32)  # one expert of up to M pairs
+    mod.set_router_bias(torch.from_numpy(bias))
+    ol = oracle.OracleLayer.from_gguf(lay.gguf, lay.config, router_bias=bias)
+    for M in (9, 17, 33, 48, 49):
+        log(f"thin layer fp16 M={M}")
+        x = lay.draw_x(M)
+        got = mod(torch.from_numpy(x).to("cuda:0")).cpu().numpy()
+        _, idx, w = ol.route(x)
+        check_forward_routing(mod, M, idx, w)
+        check_layer_output(got, ol.forward_tokens(x, idx, w))
