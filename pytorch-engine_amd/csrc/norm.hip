@@ -7,10 +7,12 @@
 // fp16 output is the MoE block's x) and model.py:1025 (attn_norm).
 //
 // One 256-thread workgroup per row; HBM-bound (x, delta, h and out streamed once, w from
-// cache), a chain of latencies at few rows.  So a thread's loads of x, delta and w all go out
-// before the first is used (per-chunk conversions by a run-time dtype had kept them in turn, and
-// w behind the barrier), and h is stored after the barrier, which would wait for it: 16 rows of
-// 2048 3.0 -> 2.6 us, 300 of 4096 5.4 -> 4.45, 4096 of 4096 (235 MB) 47.8 -> 43.6.
+// cache), a chain of latencies at few rows.  With fp32 x and delta (F32) a thread's loads of x, delta
+// and w all go out before the first is used (per-chunk conversions by a run-time dtype keep them in
+// turn, and w behind the barrier), and h is stored after the barrier, which would wait for it: 16 rows
+// of 2048 3.0 -> 2.6 us, 300 of 4096 5.4 -> 4.45, 4096 of 4096 (235 MB) 47.8 -> 43.6.  Other dtypes and
+// the plain norm load, convert and store chunk by chunk: in the F32 form, with its registers and
+// its repeats past the row, 4096 rows of fp16 took 33.8 -> 42.8 us at 5120, 69.3 -> 80.0 at 8192.
 // Thread t owns the 4-element chunks t, t + 256, ... of the row.  The sum of
 // squares has a fixed order, restated by the CPU oracle (or_add_rmsnorm): each thread adds
 // its elements' squares in element order, the 64 lanes of a wave meet by the halving tree
@@ -60,7 +62,8 @@ __device__ __forceinline__ float sq4(float acc, float4 h) {
 
 // VPT > 0: the row's chunks stay in registers (D <= 1024 * VPT); VPT == 0: the row is read
 // twice (any D), with the same order of operations.
-template <int VPT>
+// F32: x and delta are both fp32 and given (VPT > 0).
+template <int VPT, bool F32>
 __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(const void* __restrict__ x, int xdt,
                                                                   const void* __restrict__ delta, int ddt,
                                                                   const float* __restrict__ w, int D, float eps,
@@ -76,32 +79,34 @@ __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(const void* _
         return h;
     };
     float acc = 0.0f;
-    float4 hv[VPT > 0 ? VPT : 1], gv[VPT > 0 ? VPT : 1];
-    if constexpr (VPT > 0) {
+    float4 hv[VPT > 0 ? VPT : 1], gv[VPT > 0 && F32 ? VPT : 1];
+    if constexpr (VPT > 0 && F32) {
         // chunks past the row repeat its last one, so that no load is conditional
         auto at = [&](int j) { return min(t + kNormThreads * j, n4 - 1); };
-        if (delta && xdt == PGMOE_DT_F32 && ddt == PGMOE_DT_F32) {
-            float4 dv[VPT];
+        float4 dv[VPT];
 #pragma unroll
-            for (int j = 0; j < VPT; ++j) {
-                hv[j] = ((const float4*)x)[row4 + at(j)];
-                dv[j] = ((const float4*)delta)[row4 + at(j)];
-            }
-#pragma unroll
-            for (int j = 0; j < VPT; ++j) gv[j] = ((const float4*)w)[at(j)];
-            __builtin_amdgcn_sched_barrier(0);  // all of them on their way before the first is used
-#pragma unroll
-            for (int j = 0; j < VPT; ++j) hv[j] = add4(hv[j], dv[j]);
-        } else {
-#pragma unroll
-            for (int j = 0; j < VPT; ++j) {
-                gv[j] = ((const float4*)w)[at(j)];
-                hv[j] = h_at(at(j));
-            }
+        for (int j = 0; j < VPT; ++j) {
+            hv[j] = ((const float4*)x)[row4 + at(j)];
+            dv[j] = ((const float4*)delta)[row4 + at(j)];
         }
 #pragma unroll
-        for (int j = 0; j < VPT; ++j)
+        for (int j = 0; j < VPT; ++j) gv[j] = ((const float4*)w)[at(j)];
+        __builtin_amdgcn_sched_barrier(0);  // all of them on their way before the first is used
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+            hv[j] = add4(hv[j], dv[j]);
             if (t + kNormThreads * j < n4) acc = sq4(acc, hv[j]);
+        }
+    } else if constexpr (VPT > 0) {
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+            const int c = t + kNormThreads * j;
+            if (c < n4) {
+                hv[j] = h_at(c);
+                acc = sq4(acc, hv[j]);
+                if (h_out) ((float4*)h_out)[row4 + c] = hv[j];
+            }
+        }
     } else {
         for (int c = t; c < n4; c += kNormThreads) {
             const float4 h = h_at(c);
@@ -120,13 +125,16 @@ __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(const void* _
         store4(out, odt, row4 + c, make_float4((h.x * r) * g.x, (h.y * r) * g.y, (h.z * r) * g.z, (h.w * r) * g.w));
     };
     if constexpr (VPT > 0) {
-        // h is stored here too: a store before the barrier would be waited for there
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
             const int c = t + kNormThreads * j;
             if (c >= n4) continue;
-            if (h_out) ((float4*)h_out)[row4 + c] = hv[j];
-            put(c, hv[j], gv[j]);
+            if constexpr (F32) {  // h is stored here too: a store before the barrier would be waited for there
+                if (h_out) ((float4*)h_out)[row4 + c] = hv[j];
+                put(c, hv[j], gv[j]);
+            } else {
+                put(c, hv[j], ((const float4*)w)[c]);
+            }
         }
     } else {
         for (int c = t; c < n4; c += kNormThreads) put(c, h_at(c), ((const float4*)w)[c]);
@@ -138,7 +146,16 @@ int launch_add_rmsnorm(const void* x, int xdt, const void* delta, int ddt, const
     if (R == 0) return PGMOE_OK;
     const int n4 = D >> 2;
     const dim3 grid(R), block(kNormThreads);
-#define NORM(V) PG_LAUNCH(add_rmsnorm_kernel<V>, grid, block, 0, st, x, xdt, delta, ddt, w, D, eps, h_out, out, odt)
+    const bool f32 = delta && xdt == PGMOE_DT_F32 && ddt == PGMOE_DT_F32;
+#define NORM_K(V, F) \
+    PG_LAUNCH((add_rmsnorm_kernel<V, F>), grid, block, 0, st, x, xdt, delta, ddt, w, D, eps, h_out, out, odt)
+#define NORM(V)              \
+    do {                     \
+        if (f32)             \
+            NORM_K(V, true); \
+        else                 \
+            NORM_K(V, false); \
+    } while (0)
     if (n4 <= kNormThreads)
         NORM(1);
     else if (n4 <= 2 * kNormThreads)
@@ -148,8 +165,9 @@ int launch_add_rmsnorm(const void* x, int xdt, const void* delta, int ddt, const
     else if (n4 <= 8 * kNormThreads)
         NORM(8);
     else
-        NORM(0);
+        NORM_K(0, false);
 #undef NORM
+#undef NORM_K
     return check_launch("add_rmsnorm");
 }
 
