@@ -353,9 +353,12 @@ int launch_router_logits(const uint16_t* x, const float* W, const float* bias, i
         PG_ROUTER(4, 1);
     else if (M <= 8)
         PG_ROUTER(8, 1);
-    else if (!extra_w && !xsum && E >= 16 && H % 512 == 0 && H <= 4096 && (int64_t)M * E >= 24576) {
-        // the matrix-core form from 24576 logits on (fewer: its 5 us of loads and hand-over in one
-        // round outlast the vector forms; crossovers at 128 x ~170, 64 x ~450, 16 x ~1700 tokens)
+    else if (!extra_w && !xsum && E >= 16 && H % 512 == 0 && H <= 4096 &&
+             (int64_t)M * E >= (H <= 2048 ? 24576 : 32768)) {
+        // the matrix-core form from 24576 logits on, 32768 for rows of more than 2048 (fewer: its 5 us of
+        // loads and hand-over in one round outlast the vector forms; 128 experts, with the top-k: H =
+        // 2048, 192 tokens 14.2 -> 14.2 us, 384 19.7 -> 14.6; H = 4096, 192 18.3 -> 21.2, 256 21.5 ->
+        // 21.2, 288 24.4 -> 21.5)
         const int ne = div_up(E, 16), nt = div_up(M, 16);
         const dim3 grid(std::min(nt, std::max(1, 256 / ne)), ne);  // one block a CU
 #define PG_RM(J) \
@@ -376,8 +379,8 @@ int launch_router_logits(const uint16_t* x, const float* W, const float* bias, i
         PG_LAUNCH(router_gemm_kernel, dim3(div_up(M, kRgT), div_up(E, kRgE)), dim3(256), 0, st, x, W, bias, M, H, E,
                   logits);
     } else {
-        // (the LDS-tiled GEMM only from 1024 blocks: at Qwen2's M = 512 it ran 128, 18.9 us;
-        // 4 x 2 tiles 17.0 us)
+        // (the LDS-tiled GEMM, now for rows of more than 4096 values, only from 1024 blocks: 512 tokens of
+        // 3584 values and 64 experts, 128 blocks, took it 18.9 us, 4 x 2 tiles 17.0)
         // tiles of 8 tokens x 4 rows while that still makes 2048 waves; else smaller ones (the
         // shared expert's one gate row, Mixtral's 8 experts), which change no logit (each
         // (token, row) pair is summed in the same order in every tile shape).  Measured: Qwen2's

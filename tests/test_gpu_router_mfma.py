@@ -1,6 +1,7 @@
 """The matrix-core router (router_mfma_kernel): logits bit-equal to the oracle's fixed-order sums
 for every row length it takes, ragged token and expert tiles, values whose products are
-subnormal, infinities and NaN, and the calls just below its size."""
+subnormal, infinities and NaN, and the calls just below its size.  Rows of more than 4096 values take
+the LDS-tiled kernel (router_gemm_kernel) at these sizes: J = 9 and 10, ragged in tokens and experts."""
 
 import numpy as np
 import pytest
@@ -19,11 +20,15 @@ def _logits(x, w, b):
     return ops.router_topk(torch.from_numpy(x).to(dev), torch.from_numpy(w).to(dev), bt, 2, True)[0].cpu().numpy()
 
 
-# 24576 logits is the smallest call that takes it: M = 191 / 192 at 128 experts, 1445 / 1446 at 17
+# 24576 logits is the smallest call that takes it: M = 191 / 192 at 128 experts, 1445 / 1446 at 17; from
+# J = 5 on 32768: M = 511 / 512 at 64 experts, 63 / 64 at 512
 @pytest.mark.parametrize("J,E,M,bias", [(1, 128, 192, True), (2, 40, 1000, False), (3, 17, 1446, True),
                                         (3, 17, 1445, True), (4, 128, 191, False), (4, 128, 301, True),
                                         (5, 64, 385, False), (6, 512, 49, True), (7, 64, 500, False),
-                                        (8, 16, 1537, True), (4, 128, 4111, False)])
+                                        (8, 16, 1537, True), (4, 128, 4111, False), (5, 64, 511, True),
+                                        (5, 64, 512, True), (6, 512, 63, False), (6, 512, 64, True),
+                                        (7, 100, 331, False), (8, 16, 2049, True), (9, 128, 2060, True),
+                                        (10, 100, 2600, False)])
 def test_bit_exact(J, E, M, bias):
     log(f"router mfma J={J} E={E} M={M}")
     rng = np.random.default_rng(1000 * J + E + M)
