@@ -197,9 +197,10 @@ struct DenseLayout {
     size_t offsets, perm, inv, active, nact, tile_off, w, inter, isum, a16, rs, raw, total;
 };
 
-static DenseLayout dense_layout(int M, int I, int H) {
+static DenseLayout dense_layout(int M, const Mats& g, const Mats& u, const Mats& d) {
     DenseLayout o{};
-    const bool gemm = M > decode_tokens_max();
+    const int I = g.N, H = g.K;
+    const bool gemm = M > decode_tokens_max(), thin = !gemm && thin_takes_dense_decode(g, u, d, M);
     size_t c = 0;
     o.offsets = take(c, gemm ? 2 * 4 : 0);
     o.perm = take(c, gemm ? (size_t)M * 4 : 0);
@@ -210,12 +211,12 @@ static DenseLayout dense_layout(int M, int I, int H) {
     o.w = take(c, gemm ? (size_t)M * 4 : 0);
     o.inter = take(c, (size_t)M * I * 4);
     o.isum = take(c, gemm ? 0 : (size_t)M * (I / 16) * 4);
-    o.a16 = take(c, (size_t)(gemm ? M : 3 * M) * I * 2);  // decode: three rows a token
-    o.rs = take(c, (size_t)M * 4);
+    o.a16 = take(c, (size_t)(gemm ? M : thin ? 3 * M : 0) * I * 2);  // thin decode: three rows a token
+    o.rs = take(c, gemm || thin ? (size_t)M * 4 : 0);
     o.raw = take(c, gemm ? std::max(gemm_split_bytes_upto(M, 1, I, H, true), gemm_split_bytes_upto(M, 1, H, I, false))
-                         : M > 2 ? thin_dec_raw_bytes(I, H) : 0);
+                         : thin ? thin_dec_raw_bytes(I, H) : 0);
     // a workspace for many tokens serves fewer
-    o.total = gemm ? std::max(c, dense_layout(decode_tokens_max(), I, H).total) : c;
+    o.total = gemm ? std::max(c, dense_layout(decode_tokens_max(), g, u, d).total) : c;
     return o;
 }
 
@@ -244,7 +245,7 @@ extern "C" {
 size_t pgmoe_dense_workspace_bytes(const pgmoe_dense* D, int32_t M) {
     Mats g, u, d;
     if (M < 0 || check_dense(D, &g, &u, &d)) return 0;
-    return dense_layout(M, g.N, D->hidden).total;
+    return dense_layout(M, g, u, d).total;
 }
 
 int pgmoe_dense_forward(const pgmoe_dense* D, const uint16_t* x, int32_t M, float* out, void* ws, size_t ws_bytes,
@@ -256,7 +257,7 @@ int pgmoe_dense_forward(const pgmoe_dense* D, const uint16_t* x, int32_t M, floa
     if (M == 0) return PGMOE_OK;
     if (!x || !out || !ws) return fail(PGMOE_E_INVALID, "dense_forward: NULL pointer");
     if ((uintptr_t)ws & 255) return fail(PGMOE_E_INVALID, "workspace must be 256-byte aligned");
-    const DenseLayout o = dense_layout(M, g.N, D->hidden);
+    const DenseLayout o = dense_layout(M, g, u, d);
     if (ws_bytes < o.total) return fail(PGMOE_E_WORKSPACE, "workspace %zu bytes, need %zu", ws_bytes, o.total);
     uint8_t* b = (uint8_t*)ws;
 #define WS(T, f) reinterpret_cast<T*>(b + o.f)

@@ -341,3 +341,26 @@ def test_packed_linear_checks_the_member_rows():
     assert L.pgmoe_linear_forward_packed(lin, 1024, None, 0x1000, 0, 0x2000, 0, None, 0, None) == 0
     assert L.pgmoe_linear_forward_packed(None, 1, None, 0x1000, 4, 0x2000, 0, None, 0, None) == -1
     assert L.pgmoe_linear_forward(None, None, 0x1000, 4, 0x2000, 0, None, 0, None) == -1
+
+
+def test_decode_dense_workspace_holds_what_the_call_uses():
+    """The decode GEMVs use the fp32 SwiGLU rows and their 16-element sums; the split rows and sums are
+    there only for the K-quant calls of 3 and more tokens that take them, and sizes never fall."""
+    L = _lib.lib()
+    W = _lib.Weights
+
+    def dense(H, I, qt):
+        d = _lib.Dense()
+        d.hidden = H
+        d.gate, d.up, d.down = W(qt, I, H, 1, 0x100000, 0), W(qt, I, H, 1, 0x200000, 0), W(qt, H, I, 1, 0x300000, 0)
+        return d
+
+    def gemv(M, I):
+        return sum((n + 255) // 256 * 256 for n in (4 * M * I, 4 * M * (I // 16)))
+
+    for H, I, qt, first in ((4096, 12288, 12, 3), (4096, 12288, 14, 3), (4096, 12288, 8, 9), (4096, 12288, 3, 9),
+                            (4096, 8192, 1, 9), (1024, 2816, 12, 9), (2048, 5632, 13, 8)):
+        sizes = [L.pgmoe_dense_workspace_bytes(dense(H, I, qt), M) for M in range(1, 40)]
+        assert sizes == sorted(sizes)
+        for M in range(1, 9):
+            assert (sizes[M - 1] == gemv(M, I)) == (M < first), (H, I, qt, M)
