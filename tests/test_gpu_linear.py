@@ -182,3 +182,29 @@ def test_unsupported_widths_and_formats(dev):
         GGUFQuantLinear("w8", 80, 4, Q8_0, raw=np.zeros(4 * 3 * 34, np.uint8), device=dev)
     with pytest.raises(NotImplementedError):
         GGUFQuantLinear("w4", 256, 4, 16, raw=np.zeros(4 * 66, np.uint8), device=dev)  # IQ2_XXS
+
+
+@pytest.mark.parametrize("qt", [Q4_K, 13, Q6_K, Q8_0, Q4_1])
+def test_linear_past_the_thin_tiles(dev, qt):
+    """The 256-row tiles with a ragged last row and column tile and split sums, the bias and the fp16
+    rounding in the pass behind them (fewer rows take the thin tiles, which do both themselves)."""
+    lin, raw, b = _lin(qt, 1000, 4096, qt, dev, bias=True)
+    x = np.random.default_rng(qt).standard_normal((2000, 4096)).astype(np.float16)
+    log(f"linear past the thin tiles qt={qt}")
+    out = lin(torch.from_numpy(x).to(dev).float()).cpu().numpy()
+    check_layer_output(out, _ref(raw, qt, 1000, 4096, x, b, dev))
+    out16 = lin(torch.from_numpy(x).to(dev)).cpu().numpy()
+    assert np.array_equal(out16.view(np.uint16), out.astype(np.float16).view(np.uint16))
+
+
+def test_linear_rows_that_are_no_multiple_of_four(dev):
+    """Such matrices keep the 256-row tiles at any size: one super-block a row is not split, with more
+    the split sums (four columns a thread) refuse them."""
+    lin, raw, b = _lin(Q4_K, 1002, 256, 5, dev, bias=True)
+    for M in (9, 40, 300):
+        x = np.random.default_rng(M).standard_normal((M, 256)).astype(np.float16)
+        out = lin(torch.from_numpy(x).to(dev).float()).cpu().numpy()
+        check_layer_output(out, _ref(raw, Q4_K, 1002, 256, x, b, dev))
+    lin, _, _ = _lin(Q4_K, 1002, 512, 5, dev)
+    with pytest.raises(RuntimeError, match="multiple of 4"):
+        lin(torch.zeros((40, 512), dtype=torch.float16, device=dev))
