@@ -100,7 +100,8 @@ class Hip:
 
 
 # Short names of the forward's kernels (as pgmoe_moe_forward_timed reports their launches).
-_KNAMES = (("router_gemm_kernel", "router"), ("router_logits_kernel", "router"), ("topk_kernel", "topk"),
+_KNAMES = (("router_mfma_kernel", "router"), ("router_gemm_kernel", "router"),
+           ("router_logits_kernel", "router"), ("topk_kernel", "topk"),
            ("dispatch_count_kernel", "dispatch_count"), ("identity_dispatch_kernel", "sh_dispatch"),
            ("dispatch_kernel", "dispatch"), ("gemm_split_reduce_kernel<1>", "gemm_gateup_reduce"),
            ("gemm_split_reduce_kernel<0>", "gemm_down_reduce"), ("rowscale_kernel", "rowscale"),
@@ -110,15 +111,16 @@ _KNAMES = (("router_gemm_kernel", "router"), ("router_logits_kernel", "router"),
 
 
 def short_names(raw):
-    """Short labels of the launches: the products by their template's GATEUP flag; after the
-    shared expert's identity dispatch, its products (and its gate's router) get "sh_"."""
+    """Short labels of the launches: the products by their template's GATEUP flag; from the
+    shared expert's identity dispatch (its gate/up product, where that takes thin tiles) on,
+    its products (and its gate's router) get "sh_"."""
     out, shared = [], False
     for r in raw:
         if "gemm_kernel<" in r or "thin_kernel<" in r:
             n = "gemm_gateup" if ", true," in r else "gemm_down"
         else:
             n = next((v for k, v in _KNAMES if k in r), r)
-        shared = shared or n == "sh_dispatch"
+        shared = shared or n == "sh_dispatch" or (n == "gemm_gateup" and "gemm_down" in out)
         if shared and n == "router":
             n = "gate"
         out.append("sh_" + n if shared and not n.startswith("sh_") and n != "combine" else n)

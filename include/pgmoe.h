@@ -253,8 +253,8 @@ int pgmoe_moe_status(const pgmoe_layer* L, void* ws, size_t ws_bytes, int32_t* s
 size_t pgmoe_dense_workspace_bytes(const pgmoe_dense* D, int32_t M);
 
 /* One dense SwiGLU FFN: out[M, H] (fp32) = GGUFDenseMLP.forward(x[M, H]) (model.py:839-846:
- * gate||up GGUF products -> silu(gate) * up -> down).  Host-sync free and allocation free.
- * The reference's GeGLU variant (gemma) has no kernel here. */
+ * gate||up GGUF products -> act(gate) * up -> down, act SiLU or the GeGLU of gemma).
+ * Host-sync free and allocation free. */
 int pgmoe_dense_forward(const pgmoe_dense* D, const uint16_t* x, int32_t M, float* out, void* ws, size_t ws_bytes,
                         void* stream);
 
@@ -315,7 +315,8 @@ int pgmoe_dequant_rows(const pgmoe_weights* W, const int32_t* rows, int32_t n, v
  * Launch order: decode (M <= 8): gate/up (router and routing folded in), [shared gate/up,
  * shared down], down + combine (or down, combine); prefill: router, top-k, dispatch
  * (a counting pass first when it takes several workgroups), gate/up, row-scale, down,
- * [shared: identity dispatch, gate/up, row-scale, down, shared gate], combine; a product
+ * [shared: identity dispatch (if its 256-row tiles run), gate/up, row-scale, down, shared
+ * gate], combine; a product
  * split over K when its tiles cannot fill the chip is followed by its reduce kernel. */
 int pgmoe_moe_forward_timed(const pgmoe_layer* L, const uint16_t* x, int32_t M, float* out, void* ws,
                             size_t ws_bytes, void* stream, void** start_events, void** stop_events,
@@ -352,7 +353,9 @@ int pgmoe_dispatch_ws(const int32_t* topk_idx, int32_t M, int32_t K, int32_t E, 
 /* R4+R5: inter[P, I] = silu(x_p . Wg_e^T) * (x_p . Wu_e^T) for every sorted pair position p,
  * fp32 accumulate and output (gate/up_exps.forward_expert + exec_fused_act_mul_rowscale,
  * model.py:916-918).  mode 0 = wavefront GEMV (M <= 8), 1 = MFMA grouped GEMM over
- * 256-pair tiles (tile_off from pgmoe_dispatch with tile_rows = 256). */
+ * 256-pair tiles (tile_off from pgmoe_dispatch with tile_rows = 256).  pgmoe_moe_forward runs
+ * these stages too, bit for bit, except that few pairs an expert take other kernels there
+ * (sums of the same products in another order, weights rounded less). */
 int pgmoe_expert_gateup(const pgmoe_weights* gate, const pgmoe_weights* up, const uint16_t* x,
                         int32_t M, int32_t K, const int32_t* offsets, const int32_t* perm,
                         const int32_t* active, const int32_t* n_active, const int32_t* tile_off,

@@ -65,9 +65,9 @@ int launch_down(const Mats& d, const float* inter, int M, int topk, const int32_
                 const int32_t* active, const int32_t* n_active, const int32_t* tile_off, const float* topk_w,
                 int mode, uint16_t* a16, float* rs, float* partial, hipStream_t st, float* raw = nullptr,
                 const int32_t* tile_map = nullptr);
-// clear (optional): n_clear words the kernel sets to zero (the decode router's tagged logits).
 // The row-scaled fp16 down input (a16, rs) of P fp32 rows of I values.
 int launch_rowscale(const float* inter, int64_t P, int I, uint16_t* a16, float* rs, hipStream_t st);
+// clear (optional): n_clear words the kernel sets to zero (the decode router's tagged logits).
 int launch_combine(const float* partial, const int32_t* inv, int M, int K, int H, const float* shared,
                    const float* shared_logit, float* out, hipStream_t st, uint64_t* clear = nullptr,
                    int n_clear = 0);

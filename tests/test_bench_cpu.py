@@ -26,3 +26,19 @@ def test_traffic_record_resolves():
 def test_trace_average_resolves():
     us = bench.load_trace_avg("dec_gu_kernel<12, 1, 1, 2, false>")
     assert us is not None and 1.0 < us < 100.0
+
+
+def test_short_names_of_the_prefill_launches():
+    routed = ["router_mfma_kernel<4>", "(topk_kernel<4, 32>)", "dispatch_kernel"]
+    gemms = ["(gemm_kernel<QT, true, PG_GU_CT, PG_GU_WM>)", "rowscale_kernel<4>",
+             "(gemm_kernel<QT, false, PG_DN_CT, PG_DN_WM>)"]
+    thin = ["(thin_kernel<QT, true, 2, 2>)", "gemm_split_reduce_kernel<1>", "rowscale_kernel<4>",
+            "(thin_kernel<QT, false, 1, 2>)"]
+    names = ["router", "topk", "dispatch", "gemm_gateup", "rowscale", "gemm_down"]
+    assert bench.short_names(routed + gemms + ["(combine_kernel<16>)"]) == names + ["combine"]
+    shared = ["sh_gemm_gateup", "sh_rowscale", "sh_gemm_down", "sh_gate", "combine"]
+    tail = ["router_logits_kernel<1, 1>", "(combine_kernel<16>)"]
+    assert bench.short_names(routed + gemms + ["identity_dispatch_kernel"] + gemms + tail) == \
+        names + ["sh_dispatch"] + shared
+    got = bench.short_names(routed + thin + thin + tail)  # no identity dispatch in front of thin tiles
+    assert [n for n in got if "reduce" not in n] == names + shared
