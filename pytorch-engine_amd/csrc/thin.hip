@@ -17,8 +17,7 @@
 // loads stay in flight across the barriers, and 16 tokens cost 16 rows of MFMA.
 //
 // What bounds it: the weight stream.  Mixtral-shaped gate/up, 24 tokens (529 MB of Q4_K): 209
-// us on the 256-row tiles, 111-116 here (4.6-4.8 TB/s); 97 us with the loads alone (5.4 TB/s, the
-// products and decode taken out of a copy), so the VALU work is nearly hidden.  Qwen3 shape, 32
+// us on the 256-row tiles, 111-116 here (4.6-4.8 TB/s).  Qwen3 shape, 32
 // tokens: gate/up 84 -> 42 us, down 58 -> 33; H = 4096, I = 12288 FFN of 20 rows 74 -> 44 us;
 // 4096 x 6144 Q4_K linear of 33 rows 25 -> 18.6 us.  Tried and slower: two K halves in one
 // block (shorter units, no better end: 43 -> 47 us), 64-pair tiles with one row tile a wave for
@@ -901,7 +900,7 @@ int launch_thin_down(const Mats& d, const uint16_t* a16, const float* rs, int M,
 // its error against float64 falls from 2e-5 .. 3.5e-6 to 2.5e-7 .. 1.3e-7).  The GEMV decodes a
 // weight once but spends a dot2 and two LDS bytes on it for each token, so 8 tokens cost it twice
 // the weights' time; here 16 rows of MFMA cost what one does.  2048 x 151936, us GEMV -> here:
-// Q6_K 3 rows 70 -> 62, 8 rows 121 -> 64; Q4_K 56 -> 45, 103 -> 46; Q5_K 62 -> 53, 107 -> 55 (two
+// Q6_K 3 rows 65 -> 55, 8 rows 122 -> 56; Q4_K 56 -> 42, 106 -> 42; Q5_K 60 -> 48, 107 -> 49 (two
 // rows: Q6_K 60 -> 62).  Q8_0's d q is no fp16 value, so it stays there.  K is not split: from a
 // block a CU on.  The rule looks at the smallest projection of a pack, whose rows then have the
 // same bits alone and packed (gate || up of 20480 rows each stays on the GEMV, as each does).
