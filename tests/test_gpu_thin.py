@@ -304,3 +304,24 @@ def test_layer_tiles_of_fp16_experts():
         _, idx, w = ol.route(x)
         check_forward_routing(mod, M, idx, w)
         check_layer_output(got, ol.forward_tokens(x, idx, w))
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_decode_calls_keep_other_tokens_clean(bad):
+    """One token of 3 .. 8 with an infinity or NaN: the head's and the FFN's other rows are bit-equal to a
+    run without it, in the one 16-row tile and in the two that 6 and more tokens' pieces fill."""
+    from pgmoe import GGUFQuantLinear, HipDenseMLP
+    dev = torch.device("cuda", 0)
+    raw = random_blocks(np.random.default_rng(1), Q6_K, 32768, 512, 0.01)
+    head = GGUFQuantLinear("w8", 512, 32768, Q6_K, raw=raw, device=dev)
+    lay = SyntheticDense(DenseSpec("thin", 2304, 12544, (Q4_K, Q4_K, Q6_K)), seed=4, scale=0.01)
+    ffn = HipDenseMLP(lay.gguf, lay.config, 0, dev)
+    for M in (3, 5, 6, 8):
+        log(f"thin decode non-finite {bad} M={M}")
+        for call, K in ((head, 512), (ffn, 2304)):
+            x = torch.randn((M, K), generator=torch.Generator().manual_seed(M)).to(torch.float16).to(dev)
+            y = x.clone()
+            y[1, K // 3] = bad
+            clean, got = call(x), call(y)
+            keep = torch.arange(M, device=dev) != 1
+            assert torch.equal(got[keep], clean[keep]) and not torch.isfinite(got[1]).any()
