@@ -771,19 +771,22 @@ int thin_tile_rows() { return kThinTile; }
 //   up to 256 rows, where the 256-row tiles have one M tile: gate / up (two row tiles a wave) up to
 //     510 M (H = 4096, I = 12288 FFN, Q4_K: 160 rows 133 -> 112, 192 rows = 604 M 147 -> 147, 256
 //     172 -> 180; Q5_K 192 150 -> 173), else up to 850 M (28672 x 4096 Q4_K, 192 rows and 704 M 107
-//     -> 101) and 4 MB of rows, an XCD's L2 (a down product of 20480 inputs and Q4_K, 128 rows,
-//     loses 3 us of 144, one of 12288 and 192 rows 2 of 150; 4096 x 28672 Q5_K: 16 rows 49 -> 26, 64 54
-//     -> 51, 96 59 -> 71);
+//     -> 101) and 3.9 MB of rows, an XCD's L2 (with down products of 12288 inputs and 160 rows the
+//     FFN takes 107 us, 117 without; at 192 rows they lose 2 us of 150, of 13824 inputs and 144
+//     rows 5 of 160, of 20480 and 128 rows 3 of 144; 4096 x 28672 Q5_K: 16 rows 49 -> 26, 64 54 -> 51,
+//     96 59 -> 71);
 //   above, up to 450 M while those tiles leave most CUs idle (4096 x 6144 Q4_K linear, 512 rows: 86 ->
 //     57; 512 rows and more up to 150 M: 2048 x 1024 Q8_0, 1024 rows 41 -> 20, but an I = 5632 down
-//     product of 1024 rows and 369 M loses 6);
+//     product of 1024 rows and 369 M loses 6), Q5_K, the slowest to decode, up to 5 MB of rows (8192 x
+//     2048: 300 rows 43 -> 38, 384 45.5 -> 48.6);
 //   fp16 weights, which the 256-row tiles take without any decode, one tile (I = 5632 FFN: 32 rows 59 ->
 //     53, 64 rows 62 -> 64).
 bool thin_takes(int qtype, int64_t P, int N, int K, bool gateup) {
     if (N % 4 || P * K >= ((int64_t)1 << 31)) return false;  // split sums of four; 32-bit row offsets
     if (qtype == PGMOE_F16) return P <= kThinTile;
     const int64_t work = (int64_t)div_up(P, kThinTile) * N * K * (gateup ? 2 : 1);
-    if (P <= 256) return gateup ? work <= 510000000 : work <= 850000000 && P * K <= 1 << 21;
+    if (P <= 256) return gateup ? work <= 510000000 : work <= 850000000 && P * K <= 1970000;
+    if (qtype == PGMOE_Q5_K && P * K > 2500000) return false;
     return work <= (P <= 512 ? 450000000 : 150000000) && (int64_t)div_up(P, 256) * div_up(N, gateup ? 128 : 256) <= 96;
 }
 
